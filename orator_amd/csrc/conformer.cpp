@@ -5,12 +5,11 @@
 //   x += Conv(LN(x))        pointwise 2C + GLU (+ padding-row mask) in one launch, depthwise K,
 //                           BatchNorm(eval)+SiLU, pointwise C
 //   x += 0.5 FFN2(LN(x));  x = LN_out(x)
-// The projections run on the fp32 MFMA SGEMM; the attention core is either the reference
+// The projections run on the fp32 SGEMM (sgemm.hip); the attention core is either the reference
 // decomposition in fp32 (attn_mode 0) or the fused fp16 MFMA kernel (attn_mode 1).  Each
-// residual update x += s * (h W^T + b) is the last projection's epilogue or split-K reduce
-// (the same fp32 value, then one fused multiply-add, exact for s = 0.5 and 1), and that reduce
-// also writes the next block's LayerNorm of x (the closing one in place); q/k/v are one grouped
-// launch sharing LN(x).
+// residual update x += s * (h W^T + b) is the last projection's epilogue (the same fp32 value,
+// then one fused multiply-add, exact for s = 0.5 and 1), followed by the next block's LayerNorm
+// of x (the closing one in place); q/k/v are one grouped launch sharing LN(x).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -100,9 +99,8 @@ struct Conformer {
     const int P = 2 * T - 1, Dk = D / H;
     const float scale = 1.0f / std::sqrt(static_cast<float>(Dk));
     int rc = 0;
-    // FFN1.  Its LayerNorm is the only separate one: every residual update below also writes
-    // the next block's LayerNorm of x (into `ln`, whose previous contents are consumed by then;
-    // the last one, norm_out, into x itself).
+    // FFN1.  Every residual update below also writes the next block's LayerNorm of x (into `ln`,
+    // whose previous contents are consumed by then; the last one, norm_out, into x itself).
     (rc = launch_layer_norm(x, w.norm_ff1_w, w.norm_ff1_b, ln, T, D, kEps, s)) ||
         (rc = ffn(x, T, w.ff1_w1, w.ff1_b1, w.ff1_w2, w.ff1_b2, w.norm_att_w, w.norm_att_b, ln, s));
     if (rc) return rc;

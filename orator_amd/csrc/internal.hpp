@@ -198,8 +198,7 @@ int launch_sgemm_residual(const float* in, const float* W, const float* bias, fl
                           int K, int N, float res_scale, hipStream_t stream);
 
 // launch_sgemm_residual, then ln_out = LayerNorm(out rows; ln_g, ln_b, eps) (conformer_layer.cu:
-// 28-66, the next block's norm), fused into the split-K reduce when K is split and N <= 1024
-// (else a LayerNorm pass); ln_out may be out.  Same bits as the two operations.
+// 28-66, the next block's norm); ln_out may be out.
 int launch_sgemm_residual_ln(const float* in, const float* W, const float* bias, float* out,
                              int M, int K, int N, float res_scale, const float* ln_g,
                              const float* ln_b, float* ln_out, float eps, hipStream_t stream);
@@ -221,8 +220,7 @@ int launch_sgemm_group3(const float* in, const float* const W[3], const float* c
                         void* const out[3], int M, int K, int N, int h16_mask,
                         hipStream_t stream);
 
-// out[M][N] = fp16(in W^T), the fp32 product rounded to nearest even once per element (never
-// split over K): the values an fp16 consumer would round from launch_sgemm's fp32 output.
+// out[M][N] = fp16(in W^T), the fp32 product rounded to nearest even once per element: the values an fp16 consumer would round from launch_sgemm's fp32 output.
 int launch_sgemm_f16_out(const float* in, const float* W, void* out, int M, int K, int N,
                          hipStream_t stream);
 

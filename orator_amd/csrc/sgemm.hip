@@ -1,38 +1,52 @@
-// fp32 GEMM on fp32 MFMA (gfx950): out[M,N] = act(sum_k in[m,k] * W[n,k] (+ bias[n])).
+// fp32 GEMM (gfx950): out[M,N] = act(sum_k in[m,k] * W[n,k] (+ bias[n])).
 //
 // Replaces gemm::LaunchSgemm / LaunchSgemmBatched (include/model/gemm.cuh:47-268): the same
 // nn.Linear "NT" contract (both operands K-contiguous), activation codes 0 none, 1 SiLU,
-// 2 ReLU, 3 sigmoid (gemm.cuh:38-45), strided batches, arbitrary M/N/K and alignment
-// (guarded loads, as SgemmBatchedKernel).  Products are exact fp32 and accumulate in fp32
-// on v_mfma_f32_32x32x2_f32, so results stay within fp32 rounding of the reference's
-// k-sequential FMA chains.
+// 2 ReLU, 3 sigmoid (gemm.cuh:38-45), strided batches, arbitrary M/N/K and alignment.
 //
-// Workgroup = 64 x 64 tile of one batch entry, 4 waves of one 32 x 32 block each, four
-// workgroups per CU (fp32 MFMA is 16x slower per flop than bf16, so these small products are
-// latency-bound and want many resident waves, not big tiles: 128 x 128 tiles measured 1.6-2.8x
-// slower at the Conformer's shapes).  K advances 32 floats at a time through two LDS buffers
-// (rows padded to 36 floats = 144 bytes: the 16 rows a quarter-wave reads land on distinct
-// 16-byte bank groups).  MFMA k-step j takes k = 2j from the lower half-wave and 2j + 1 from
-// the upper (the pairs in k order, as a k-sequential chain adds them); LDS rows hold the even k
-// then the odd k, so one ds_read_b128 per lane still feeds four MFMAs.  The next K tile is
-// loaded into registers while the current one is multiplied and stored before the step's last
-// MFMAs, the next fragments are read under the current ones; one barrier per step.  When the
-// grid leaves CUs idle and K is long, K is split over workgroups and the partials are summed
-// in a fixed order.
+// fp32 products on the bf16 matrix cores: every operand is split in registers into three bf16
+// terms whose sum is the fp32 value exactly, and the six products of terms that reach fp32's
+// precision are accumulated in fp32 (what is dropped is below 2^-26 of |x w|, and the MFMA adds
+// 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96 cycles
+// per 16 x 16 x 32 block, the fp32 MFMA's 256.  Measured against 64 bits (random normal
+// operands, relative 2-norm): K = 512 0.8-1.2e-7, K = 2048 1.7e-7, K = 64 4.7e-8; the fp32 MFMA
+// 2.9e-7 unsplit (2.1e-7 with K in two parts), 2.1e-7 in eight parts, 1.4e-7.
+//
+// Workgroup = BM x BN tile of one batch entry; its WK waves share the tile and split K: wave w
+// takes the 32-float slices w, w + WK, ..., accumulates the whole tile in registers, and the WK
+// partial tiles are added in LDS in wave order (deterministic).  So every element is loaded and
+// split by exactly one wave of the workgroup, and the k loop has no barrier: a wave's slice comes
+// by buffer loads straight into the wave's own LDS area (8 lanes per 128-byte row piece; read as
+// fragments directly from memory, 16 rows per instruction, the same loads ran at 16 bytes per
+// clock and CU), goes to registers whole, and the next slice's loads run under the MFMAs.  What
+// bounds it: the splitting (about 3.7 VALU instructions per MFMA at 64 x 64) and the MFMAs share
+// the issue slots -- a slice of a 64 x 64 tile takes ~2700 cycles per SIMD against 1536 of MFMA
+// alone, with the loads removed 9 % less -- and, at the Conformer's sizes, the ~4 us of launch,
+// first loads and epilogue.  The bf16 dot product in place of the unpack + subtraction saves a
+// fifth of the VALU work but occupies the matrix cores: no faster.  Interleaving VALU and MFMA by
+// scheduling groups and wave priorities: no effect.
+//
+// Measured (us, replayed launches; before: the fp32-MFMA kernel with split K and its reduction):
+//   717 x 512 -> 2048  28.7 -> 16.3   717 x 2048 -> 512  24.5 -> 17.3   717 x 512 -> 512 12.2 -> 8.2
+//   717 x 512 -> 1536  27.0 -> 15.1   1433 x 512 -> 512  15.4 -> 10.6   717 x 512 -> 1024 15.4 -> 10.8
+//   126 x 512 -> 2048  11.2 -> 5.9    126 x 2048 -> 512  12.7 -> 11.9   126 x 512 -> 512 10.3 -> 5.8
+//   8 x (717 x 717 -> 64) 19.8 -> 13.5; 8 x (717 x 64 -> 717) 14.2 -> 14.1, 8 x (1000 x 64 -> 1999)
+//   31.2 -> 36.6 (bound by its 64 MB of unaligned rows written).
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "mfma_tile.hpp"
 
 namespace orator_hip {
 namespace {
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kSK = 32;        // K per step (floats)
-constexpr int kSLd = kSK + 4;  // padded LDS row
+constexpr int kSK = 32;  // K per slice (floats)
 
 __device__ __forceinline__ float apply_act(float v, int act) {
   if (act == 1) return v / (1.0f + expf(-v));
@@ -46,9 +60,8 @@ struct SgemmArgs {
   const float* W;
   const float* bias;
   float* out;
-  float* part;  // split-K partials [splits][batch][M][N], or nullptr
-  int M, K, N, act, k_split;
-  int batch, splits;  // blockIdx.z = split * batch + batch entry
+  int M, K, N, act;
+  int batch;  // blockIdx.z = batch entry
   long s_in, s_w, s_out;
   bool vec;  // K % 32 == 0 and 16-byte aligned operands: 16-byte loads
   // Grouped products (group > 0): `group` problems share `in`; problem z uses weight Wg[z],
@@ -60,201 +73,220 @@ struct SgemmArgs {
   // Residual update (residual != 0): out = out + res_scale * (in W^T + bias), act 0.
   int residual;
   float res_scale;
-  // GLU (the kSEpiGlu epilogue): W has 2 glu_c rows (value rows, then gate rows); out[m][c] =
+  // GLU (the GLU epilogue): W has 2 glu_c rows (value rows, then gate rows); out[m][c] =
   // a * (1 / (1 + exp(-b))) with a, b the value and gate outputs (bias added), 0 for rows
   // m >= glu_valid; out is [M][glu_c].
   int glu_c, glu_valid;
-  // LayerNorm of the updated rows (ln_g non-null; split-K reduce only): ln_out[m] =
-  // (x - mean) rsqrt(var + eps) g + b over the row's N values x = out[m] after the residual
-  // update; ln_out == out writes the normalised row only.
+  // LayerNorm of the updated rows (ln_g non-null), a launch of its own after the product:
+  // ln_out[m] = LayerNorm(out[m]) g + b; ln_out may be out.
   const float* ln_g;
   const float* ln_b;
   float* ln_out;
   float ln_eps;
+  bool chain;  // every output as one fp32 chain (rows too long for 32-bit tile offsets)
   // fp16 outputs: bit z set stores problem z's output (group products; bit 0 otherwise) as
-  // fp16, each value rounded to nearest even once; unsplit products without residual only.
+  // fp16, each value rounded to nearest even once; products without residual only.
   int h16;
 };
 
-// Epilogues: raw split-K partials, out = acc (no bias, act 0), and through LDS out =
-// act(acc + bias) or the residual update out += res_scale * (acc + bias), or the GLU of a
-// tile's value and gate halves.  out = acc and out = act(acc + bias) may be stored as fp16 (h16).
-constexpr int kSEpiPartial = 0, kSEpiStore = 1, kSEpiAct = 2, kSEpiGlu = 3;
+// Eight fp32 values as three bf16 terms each, x = h + m + l exactly (8 + 8 + 8 significant
+// bits, each term the rest rounded to nearest).
+struct Split {
+  bf16x8_t h, m, l;
+};
+__device__ __forceinline__ Split split_bf16x3(float4 u, float4 v) {
+  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    h[w] = cvt_bf16x2(x[2 * w], x[2 * w + 1]);
+    const float r0 = x[2 * w] - bf16_lo(h[w]), r1 = x[2 * w + 1] - bf16_hi(h[w]);
+    m[w] = cvt_bf16x2(r0, r1);
+    l[w] = cvt_bf16x2(r0 - bf16_lo(m[w]), r1 - bf16_hi(m[w]));
+  }
+  return {as_bf16x8(make_uint4(h[0], h[1], h[2], h[3])),
+          as_bf16x8(make_uint4(m[0], m[1], m[2], m[3])),
+          as_bf16x8(make_uint4(l[0], l[1], l[2], l[3]))};
+}
 
-template <int BM, int BN, int WGM, int WGN, int MINW, bool VEC, int EPI>
-__global__ __launch_bounds__(64 * WGM * WGN, MINW) void sgemm_nt_kernel(SgemmArgs a) {
-  constexpr int NT = 64 * WGM * WGN;
-  constexpr int TM = BM / WGM, TN = BN / WGN;
-  constexpr int FM = TM / 32, FN = TN / 32;
-  constexpr int RPI = NT / 8;  // rows per load instruction (8 threads x 16 bytes per row)
-  // load instructions per thread per K step; a tile side that is not a multiple of RPI (96 x 64
-  // tiles: 48 rows per instruction) loads clamped rows past it and does not store them
-  constexpr int LA = (BM + RPI - 1) / RPI, LW = (BN + RPI - 1) / RPI;
-  // LDS: the double-buffered tiles during the K loop, then (bias / activation epilogue) the
-  // fp32 output tile, rows padded by 8 floats
-  constexpr int kCLd = BN + 8;
-  constexpr int kTileBytes = 2 * (BM + BN) * kSLd * 4;
-  constexpr int kOutBytes = BM * kCLd * 4;
-  __shared__ __align__(16) unsigned char smem[kTileBytes > kOutBytes ? kTileBytes : kOutBytes];
-  auto sA = reinterpret_cast<float(*)[BM][kSLd]>(smem);
-  auto sW = reinterpret_cast<float(*)[BN][kSLd]>(smem + 2 * BM * kSLd * 4);
-  auto sC = reinterpret_cast<float(*)[kCLd]>(smem);
+template <int BM, int BN, int WK, bool VEC, bool GLU>
+__global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
+  constexpr int NT = 64 * WK;
+  constexpr int FM = BM / 16, FN = BN / 16;
+  // per wave: a slice of BM + BN rows of 128 bytes while k runs, then its fp32 output tile (rows
+  // padded by 4 floats: the 16 rows a quarter-wave writes 16 bytes of land on distinct bank
+  // groups)
+  constexpr int kCLd = BN + 4;
+  constexpr int kSliceFloats = (BM + BN) * kSK, kTileFloats = BM * kCLd;
+  constexpr int kWaveFloats = kSliceFloats > kTileFloats ? kSliceFloats : kTileFloats;
+  __shared__ __align__(16) float smem[WK][kWaveFloats];
 
-  const int batch = blockIdx.z % a.batch;
-  const int split = blockIdx.z / a.batch;
+  // Workgroups are dealt to the 8 XCDs in turn: give each a contiguous piece of the tile order
+  // (batch entries, then tiles with the operand of more rows running slowest), so the tiles that
+  // share an L2 share rows of it, and the lines that neighbours write in part meet there.
+  const int gx = gridDim.x, gy = gridDim.y, total_wg = gx * gy * static_cast<int>(gridDim.z);
+  const int lin = blockIdx.x + gx * (blockIdx.y + gy * static_cast<int>(blockIdx.z));
+  const int xcd = lin & 7;
+  const int at = xcd * (total_wg >> 3) + min(xcd, total_wg & 7) + (lin >> 3);
+  const int batch = at / (gx * gy), in_batch = at - batch * (gx * gy);
+  const bool n_slow = a.N > a.M;
+  const int tile_n = n_slow ? in_batch / gy : in_batch % gx;
+  const int tile_m = n_slow ? in_batch % gy : in_batch / gx;
   const float* A = a.in + batch * a.s_in;
   const float* B = a.group ? a.Wg[batch] : a.W + batch * a.s_w;
   const int M = a.M, N = a.N, K = a.K;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / WGN, wn = wave % WGN;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int kb = split * a.k_split;
-  const int k_end = min(K, kb + a.k_split);
-  const int lr = tid >> 3, lc = tid & 7;
-  // 16-byte loads (VEC: K a multiple of the 32-float step, 16-byte aligned operands, so every
-  // split is whole steps): rows clamped into range (their outputs are never stored), no
-  // branches.  Otherwise guarded scalar loads.
-  const float* arow[LA];
-  const float* wrow[LW];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  // GLU: tile rows [0, BN/2) are value rows from c0 on, [BN/2, BN) the matching gate rows
+  constexpr int BW = GLU ? BN / 2 : BN;  // rows of one block of W rows
+  const int w0 = tile_n * BW, w_last = (GLU ? a.glu_c : N) - 1;
+  // Rows behind tile rows, clamped into range (outputs past M and N are never stored)
+  auto a_row = [&](int t) { return A + static_cast<long>(min(m0 + t, M - 1)) * K; };
+  auto w_row = [&](int t) {
+    const long r = min(w0 + t % BW, w_last) + (t >= BW ? a.glu_c : 0);
+    return B + r * K;
+  };
+  // the slice's rows through buffer loads straight into LDS; offsets count from the tile's
+  // first row, so they fit 32 bits whatever the matrix's size
+  const uint32_t row_bytes = static_cast<uint32_t>(K) * 4;
+  auto rsrc = [&](const float* p, int rows) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, rows * row_bytes,
+                                             0x00020000);
+  };
+  const int rows_a = min(BM, M - m0), rows_w = min(BW, w_last + 1 - w0);
+  const __amdgpu_buffer_rsrc_t rs_a = rsrc(A + static_cast<long>(m0) * K, rows_a);
+  const __amdgpu_buffer_rsrc_t rs_w = rsrc(B + static_cast<long>(w0) * K, rows_w);
+  const __amdgpu_buffer_rsrc_t rs_g =
+      GLU ? rsrc(B + (static_cast<long>(a.glu_c) + w0) * K, rows_w) : rs_w;
+  // LDS row = 8 chunks of 16 bytes, chunk c in slot c ^ swz(row): fragment reads (16 rows, one
+  // chunk) then hit distinct banks
+  auto swz = [](int row) { return (row & 7) ^ ((row >> 3) & 1); };
+  float* const mine = smem[wave];
+  auto dma = [&](int s) {
+    // VEC: 8 rows per instruction, 8 lanes x 16 bytes each; else 2 rows, 32 lanes x 4 bytes,
+    // elements past K as zeros (an offset past the buffer)
+    constexpr int RPI = VEC ? 8 : 2, LPR = 64 / RPI;
 #pragma unroll
-  for (int i = 0; i < LA; ++i) arow[i] = A + static_cast<long>(min(m0 + RPI * i + lr, M - 1)) * K;
-#pragma unroll
-  for (int i = 0; i < LW; ++i) {
-    if constexpr (EPI == kSEpiGlu) {  // tile rows: BN/2 value rows, then the matching gate rows
-      const int t = RPI * i + lr, c = blockIdx.x * (BN / 2) + (t % (BN / 2));
-      wrow[i] = B + static_cast<long>((t < BN / 2 ? 0 : a.glu_c) + min(c, a.glu_c - 1)) * K;
-    } else {
-      wrow[i] = B + static_cast<long>(min(n0 + RPI * i + lr, N - 1)) * K;
+    for (int q = 0; q < (BM + BN) / RPI; ++q) {
+      const int t = q * RPI;  // tile row of the instruction: A rows, then W rows
+      const bool is_a = t < BM;
+      const int first = is_a ? t : (t - BM) % BW;
+      const int r = first + lane / LPR;
+      const int row = min(r, (is_a ? rows_a : rows_w) - 1);
+      const int lds_row = t + lane / LPR;
+      uint32_t off, soff = 0;
+      if constexpr (VEC) {
+        off = row * row_bytes + 16 * ((lane % LPR) ^ swz(lds_row));
+        soff = static_cast<uint32_t>(s) * (kSK * 4);
+      } else {
+        const int e = lane % LPR, k = s * kSK + 4 * ((e >> 2) ^ swz(lds_row)) + (e & 3);
+        off = k < K ? row * row_bytes + 4 * k : 0xfffffffcu;
+      }
+      const __amdgpu_buffer_rsrc_t rs = is_a ? rs_a : t - BM < BW ? rs_w : rs_g;
+      const auto dst = (__attribute__((address_space(3))) void*)(mine + t * kSK);
+      if constexpr (VEC)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 16, off, soff, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, off, soff, 0, 0);
     }
-  }
-  float4 ra[LA], rw[LW];
-  auto load_guarded = [&](const float* base, int row, int rows, int k) -> float4 {
-    if (row >= rows) return make_float4(0.f, 0.f, 0.f, 0.f);
-    const float* p = base + static_cast<long>(row) * K + k;
-    float4 v;
-    v.x = k < k_end ? p[0] : 0.f;
-    v.y = k + 1 < k_end ? p[1] : 0.f;
-    v.z = k + 2 < k_end ? p[2] : 0.f;
-    v.w = k + 3 < k_end ? p[3] : 0.f;
-    return v;
   };
-  auto load = [&](int k0) {
-    const int k = k0 + 4 * lc;
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const float4*>(arow[i] + k);
-#pragma unroll
-      for (int i = 0; i < LW; ++i) rw[i] = *reinterpret_cast<const float4*>(wrow[i] + k);
-    } else {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = load_guarded(A, m0 + RPI * i + lr, M, k);
-#pragma unroll
-      for (int i = 0; i < LW; ++i) rw[i] = load_guarded(B, n0 + RPI * i + lr, N, k);
-    }
-  };
-  // LDS row = [even k | odd k]: k = 4c..4c+3 of a 16-byte load go to slots 2c, 2c+1 of each
-  // half, so a lane of half h reading slots 4q..4q+3 of half h gets k = 2j + h, j = 4q..4q+3
-  auto put = [&](float* row, float4 v) {
-    *reinterpret_cast<float2*>(row + 2 * lc) = make_float2(v.x, v.z);
-    *reinterpret_cast<float2*>(row + 16 + 2 * lc) = make_float2(v.y, v.w);
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < LA; ++i)
-      if (BM % RPI == 0 || RPI * i + lr < BM) put(&sA[buf][RPI * i + lr][0], ra[i]);
-#pragma unroll
-    for (int i = 0; i < LW; ++i)
-      if (BN % RPI == 0 || RPI * i + lr < BN) put(&sW[buf][RPI * i + lr][0], rw[i]);
-  };
-
-  f32x16_t acc[FM][FN];
+  // Fragment: lane = (row lane % 16, group lane / 16); group g takes floats 4g .. 4g + 3 and
+  // 16 + 4g .. of the slice (the same k for A and W, so any assignment serves)
+  const int fr = lane & 15, fg = lane >> 4;
+  f32x4_t acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int fr = lane & 31, fk = 16 * (lane >> 5);
-  const int n_k = (k_end - kb + kSK - 1) / kSK;
-  load(kb);
-  store(0);
-  lds_barrier();
-  for (int t = 0; t < n_k; ++t) {
-    const int buf = t & 1;
-    if (t + 1 < n_k) load(kb + (t + 1) * kSK);
-    float4 fa[2][FM], fb[2][FN];
-    auto read = [&](int q, int s) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-        fa[s][i] = *reinterpret_cast<const float4*>(&sA[buf][wm * TM + 32 * i + fr][fk + 4 * q]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        fb[s][j] = *reinterpret_cast<const float4*>(&sW[buf][wn * TN + 32 * j + fr][fk + 4 * q]);
+  const int n_sl = a.chain ? 0 : (K + kSK - 1) / kSK;
+  if (wave < n_sl) dma(wave);
+  for (int s = wave; s < n_sl; s += WK) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // The whole slice to registers as bf16 terms, then the next slice's loads under the MFMAs:
+    // the six products of terms that reach fp32's precision (the dropped m l, l m and l l are
+    // below 2^-26 of |x w|), smallest first.  The W fragment is the MFMA's row operand, so a
+    // lane ends up with 4 consecutive columns of one output row.
+    float4 raw_a[FM][2], raw_w[FN][2];
+    auto fetch = [&](float4(&raw)[2], int t) {
+      const float* row = mine + (t + fr) * kSK;
+      const int x = swz(t + fr);
+      raw[0] = *reinterpret_cast<const float4*>(row + 4 * (fg ^ x));
+      raw[1] = *reinterpret_cast<const float4*>(row + 4 * ((4 + fg) ^ x));
     };
-    read(0, 0);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int s = q & 1;
-      if (q + 1 < 4) read(q + 1, s ^ 1);  // next fragments under this q's MFMAs
-      // the next tile goes to the other (idle) buffer before the step's last MFMAs
-      if (q == 3 && t + 1 < n_k) store(buf ^ 1);
+    for (int j = 0; j < FN; ++j) fetch(raw_w[j], BM + 16 * j);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+    for (int i = 0; i < FM; ++i) fetch(raw_a[i], 16 * i);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (s + WK < n_sl) dma(s + WK);
+    Split sa[FM];
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] =
-                __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s][i][e], fb[s][j][e], acc[i][j], 0, 0, 0);
-    }
-    lds_barrier();
-  }
-
-  // block (i, j): lane holds column 32 j + lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4
-  // of the block.  Plain stores and partials go straight out (nothing is loaded, so no store
-  // waits); bias / activation go through LDS with the bias loaded before the first store
-  // (stores count against the same wait counter as loads).
-  if constexpr (EPI == kSEpiPartial || EPI == kSEpiStore) {
-    float* C = EPI == kSEpiPartial
-                   ? a.part + (static_cast<long>(split) * a.batch + batch) * M * N
-                   : (a.group ? a.og[batch] : a.out + batch * a.s_out);
+    for (int i = 0; i < FM; ++i) sa[i] = split_bf16x3(raw_a[i][0], raw_a[i][1]);
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      const int n = n0 + wn * TN + 32 * j + fr;
-      if (n >= N) continue;
+      const Split w = split_bf16x3(raw_w[j][0], raw_w[j][1]);
+      auto mma = [&](const bf16x8_t& x, auto term) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * TM + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-          if (m >= M) continue;
-          if (EPI == kSEpiStore && (a.h16 & 1))  // ungrouped: bit 0
-            reinterpret_cast<_Float16*>(C)[static_cast<long>(m) * N + n] =
-                static_cast<_Float16>(acc[i][j][e]);
-          else
-            C[static_cast<long>(m) * N + n] = acc[i][j][e];
-        }
+        for (int i = 0; i < FM; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, sa[i].*term, acc[i][j], 0, 0, 0);
+      };
+      mma(w.l, &Split::h);
+      mma(w.h, &Split::l);
+      mma(w.m, &Split::m);
+      mma(w.m, &Split::h);
+      mma(w.h, &Split::m);
+      mma(w.h, &Split::h);
     }
-    return;
   }
+
+  // Per-wave partial tiles to LDS, then the sum over the waves (in wave order) and the
+  // epilogue, a thread per 4 columns
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        sC[wm * TM + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)][wn * TN + 32 * j + fr] =
-            acc[i][j][e];
+      *reinterpret_cast<f32x4_t*>(mine + (16 * i + fr) * kCLd + 16 * j + 4 * fg) = acc[i][j];
   __syncthreads();
-  if constexpr (EPI == kSEpiGlu) {
+  // A value that is not finite (an infinite or NaN operand, one that rounds past bf16's range,
+  // an overflow), or so small that operands below 2^-109, whose third terms fall between bf16's
+  // subnormal numbers, may be behind it, is formed again as one fp32 chain.
+  auto suspect = [&](float t) {
+    const float mag = fabsf(t);
+    return !(mag < INFINITY) || (mag < 0x1p-90f && mag != 0.0f) || a.chain;
+  };
+  auto chain = [&](int r, int c) {
+    const float* x = a_row(r);
+    const float* y = w_row(c);
+    float t = 0.0f;
+#pragma unroll 8
+    for (int k = 0; k < K; ++k) t = fmaf(x[k], y[k], t);
+    return t;
+  };
+  auto total = [&](int r, int c, float (&v)[4]) {
+    f32x4_t t = *reinterpret_cast<const f32x4_t*>(smem[0] + r * kCLd + c);
+#pragma unroll
+    for (int w = 1; w < WK; ++w) t += *reinterpret_cast<const f32x4_t*>(smem[w] + r * kCLd + c);
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[q] = t[q];
+      any |= suspect(t[q]);
+    }
+    if (any) [[unlikely]] {
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q)
+        if (suspect(v[q])) v[q] = chain(r, c + q);
+    }
+  };
+  if constexpr (GLU) {
     // columns [0, BN/2) of the tile are the value outputs of channels c0 .., [BN/2, BN) the
     // gate outputs of the same channels; the same fp32 values and formula as a plain product
     // followed by the GLU pass (its bias added, then a * (1 / (1 + exp(-b))))
-    constexpr int HB = BN / 2, TPRg = HB / 4, RPIg = NT / TPRg, PASSES_G = BM / RPIg;
-    const int Cg = a.glu_c, c0 = blockIdx.x * HB;
+    constexpr int HB = BN / 2, TPRg = HB / 4, RPIg = NT / TPRg;
+    const int Cg = a.glu_c, c0 = tile_n * HB;
     const int orow = tid / TPRg, j = 4 * (tid % TPRg);
     float ba[4] = {0.f, 0.f, 0.f, 0.f}, bg[4] = {0.f, 0.f, 0.f, 0.f};
     if (a.bias) {
@@ -265,20 +297,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void sgemm_nt_kernel(SgemmArg
       }
     }
     const bool vec_out = (Cg % 4) == 0 && ((reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-#pragma unroll
-    for (int p = 0; p < PASSES_G; ++p) {
-      const int r = RPIg * p + orow;
+    for (int r = orow; r < BM; r += RPIg) {
       const int m = m0 + r;
-      const float4 va = *reinterpret_cast<const float4*>(&sC[r][j]);
-      const float4 vg = *reinterpret_cast<const float4*>(&sC[r][HB + j]);
-      const float av[4] = {va.x, va.y, va.z, va.w}, gv[4] = {vg.x, vg.y, vg.z, vg.w};
-      float o[4];
+      if (m >= M) continue;
+      float av[4], gv[4], o[4];
+      total(r, j, av);
+      total(r, HB + j, gv);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float x = av[q] + ba[q], g = gv[q] + bg[q];
         o[q] = m < a.glu_valid ? x * (1.0f / (1.0f + __expf(-g))) : 0.0f;
       }
-      if (m >= M) continue;
       float* dst = a.out + static_cast<long>(m) * Cg + c0 + j;
       if (vec_out && c0 + j + 3 < Cg) {
         *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
@@ -293,236 +322,121 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void sgemm_nt_kernel(SgemmArg
   float* C = a.group ? a.og[batch] : a.out + batch * a.s_out;
   const float* bias = a.group ? a.bg[batch] : a.bias;
   const bool h16 = (a.h16 >> (a.group ? batch : 0)) & 1;
-  constexpr int TPRo = BN / 4, RPIo = NT / TPRo, PASSES = BM / RPIo;
-  const int orow = tid / TPRo, ocol = 4 * (tid % TPRo);
-  const int n = n0 + ocol;
-  const bool vec_out = (N % 4) == 0 && ((reinterpret_cast<uintptr_t>(C)) & 15) == 0;
-  const bool vec_h16 = (N % 4) == 0 && ((reinterpret_cast<uintptr_t>(C)) & 7) == 0;
-  float bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias) {
+  auto finish = [&](float v, float b, const float* old) {
+    v = apply_act(v + b, a.act);
+    return a.residual ? fmaf(a.res_scale, v, *old) : v;
+  };
+  if ((N % 4) == 0 && (reinterpret_cast<uintptr_t>(C) & (h16 ? 7 : 15)) == 0) {
+    // 4 columns per thread, one 16-byte (fp16: 8-byte) store
+    constexpr int TPRo = BN / 4, RPIo = NT / TPRo;
+    const int orow = tid / TPRo, ocol = 4 * (tid % TPRo);
+    const int n = n0 + ocol;
+    if (n >= N) return;
+    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (bias) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) bv[q] = bias[min(n + q, N - 1)];
-  }
-  // the residual's old values, all loaded before the first store
-  float old[PASSES][4];
-  if (a.residual) {
-#pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-      const float* src = C + static_cast<long>(min(m0 + RPIo * p + orow, M - 1)) * N;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) old[p][q] = src[min(n + q, N - 1)];
+      for (int q = 0; q < 4; ++q) bv[q] = bias[n + q];
     }
-  }
+    for (int r = orow; r < BM && m0 + r < M; r += RPIo) {
+      const long at = static_cast<long>(m0 + r) * N + n;
+      float v[4];
+      total(r, ocol, v);
 #pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-    const int r = RPIo * p + orow;
-    const int m = m0 + r;
-    const float4 c = *reinterpret_cast<const float4*>(&sC[r][ocol]);
-    float v[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      v[q] = apply_act(v[q] + bv[q], a.act);
-      if (a.residual) v[q] = fmaf(a.res_scale, v[q], old[p][q]);
-    }
-    if (m >= M) continue;
-    if (h16) {
-      _Float16* dst = reinterpret_cast<_Float16*>(C) + static_cast<long>(m) * N + n;
-      if (vec_h16 && n + 3 < N) {
+      for (int q = 0; q < 4; ++q) v[q] = finish(v[q], bv[q], C + at + q);
+      if (h16) {
         typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
         const h4_t hv = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]),
                          static_cast<_Float16>(v[2]), static_cast<_Float16>(v[3])};
-        *reinterpret_cast<h4_t*>(dst) = hv;
+        *reinterpret_cast<h4_t*>(reinterpret_cast<_Float16*>(C) + at) = hv;
       } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (n + q < N) dst[q] = static_cast<_Float16>(v[q]);
+        *reinterpret_cast<float4*>(C + at) = make_float4(v[0], v[1], v[2], v[3]);
       }
-      continue;
     }
-    float* dst = C + static_cast<long>(m) * N + n;
-    if (vec_out && n + 3 < N) {
-      *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
+    return;
+  }
+  // other row lengths and alignments: a column per thread, so that a store instruction still
+  // writes whole row pieces
+  constexpr int RPS = NT / BN;  // rows per pass
+  const int c = tid % BN, n = n0 + c;
+  if (n >= N) return;
+  const float b = bias ? bias[n] : 0.0f;
+  constexpr int U = BM / RPS < 4 ? BM / RPS : 4;
+  for (int r0 = tid / BN; r0 < BM && m0 + r0 < M; r0 += U * RPS) {
+    float v[U];
+    bool any = false;
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (n + q < N) dst[q] = v[q];
+    for (int u = 0; u < U; ++u) {
+      const int r = r0 + u * RPS;
+      v[u] = smem[0][r * kCLd + c];
+#pragma unroll
+      for (int w = 1; w < WK; ++w) v[u] += smem[w][r * kCLd + c];
+      any |= suspect(v[u]);
+    }
+    if (any) [[unlikely]] {
+#pragma unroll 1
+      for (int u = 0; u < U; ++u)
+        if (suspect(v[u])) v[u] = chain(r0 + u * RPS, c);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int m = m0 + r0 + u * RPS;
+      if (m >= M) break;
+      const long at = static_cast<long>(m) * N + n;
+      const float x = finish(v[u], b, C + at);
+      if (h16)
+        reinterpret_cast<_Float16*>(C)[at] = static_cast<_Float16>(x);
+      else
+        C[at] = x;
     }
   }
 }
 
-// out_b[m][n] = act(sum_z part[z][b][m][n] + bias[n]), z ascending (a fixed order).
-__global__ __launch_bounds__(256) void sgemm_splitk_reduce_kernel(const float* __restrict__ part,
-                                                                  int splits, int batch,
-                                                                  const float* __restrict__ bias,
-                                                                  float* __restrict__ out, int M,
-                                                                  int N, int act, long s_out,
-                                                                  int residual, float res_scale) {
-  const long MN = static_cast<long>(M) * N;
-  const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= MN * batch) return;
-  const long b = i / MN, r = i - b * MN;
-  const long per_split = MN * batch;
-  float v = part[i];
-  for (int z = 1; z < splits; ++z) v += part[z * per_split + i];
-  v = apply_act(v + (bias ? bias[r % N] : 0.0f), act);
-  if (residual) v = fmaf(res_scale, v, out[b * s_out + r]);
-  out[b * s_out + r] = v;
+template <int BM, int BN, int WK, bool VEC, bool GLU>
+int launch_tile(const SgemmArgs& a, hipStream_t s) {
+  const int bn = GLU ? BN / 2 : BN, cols = GLU ? a.glu_c : a.N;
+  const dim3 grid((cols + bn - 1) / bn, (a.M + BM - 1) / BM, a.batch);
+  hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WK, VEC, GLU>), grid, dim3(64 * WK), 0, s, a);
+  return check_launch("sgemm_nt_kernel");
 }
 
-// The split-K reduce with the residual update, then a LayerNorm of each updated row: one wave
-// per row, lane l holding columns l, l + 64, ... (N <= 64 PER).  Per element the same
-// arithmetic as sgemm_splitk_reduce_kernel (partials in split order, bias, residual fmaf);
-// the normalisation is layer_norm_kernel's (lane-order sums, the wave sum, contraction off),
-// so x and LN(x) carry the same bits as the reduce followed by the LayerNorm pass.
-constexpr int kMaxLnSplits = 8;  // the split count run_sgemm chooses is at most 8
-
-template <int PER, int MAXS>
-__global__ __launch_bounds__(256) void sgemm_splitk_reduce_ln_kernel(
-    const float* __restrict__ part, int splits, const float* __restrict__ bias, float* out,
-    int M, int N, float res_scale, const float* __restrict__ g, const float* __restrict__ b,
-    float* ln_out, float eps) {
-#pragma clang fp contract(off)
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= M) return;
-  const long MN = static_cast<long>(M) * N;
-  const long base = static_cast<long>(row) * N;
-  // every partial of the lane's columns is loaded at once (one memory round trip: a wave per
-  // row leaves few waves per CU); the sum keeps split order, terms past `splits` selected away
-  float p[PER][MAXS], old[PER], bv[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int n = min(lane + 64 * i, N - 1);
-#pragma unroll
-    for (int z = 0; z < MAXS; ++z) p[i][z] = part[min(z, splits - 1) * MN + base + n];
-    old[i] = out[base + n];
-    bv[i] = bias ? bias[n] : 0.0f;
-  }
-  float v[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    float x = p[i][0];
-#pragma unroll
-    for (int z = 1; z < MAXS; ++z) x = z < splits ? x + p[i][z] : x;
-    x = x + bv[i];
-    v[i] = fmaf(res_scale, x, old[i]);
-  }
-  const bool in_place = ln_out == out;
-#pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (!in_place && lane + 64 * i < N) out[base + lane + 64 * i] = v[i];
-  float sum = 0.0f;
-#pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (lane + 64 * i < N) sum += v[i];
-  const float mean = wave_sum(sum) / static_cast<float>(N);
-  float sq = 0.0f;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const float t = v[i] - mean;
-    if (lane + 64 * i < N) sq += t * t;
-  }
-  const float inv = rsqrtf(wave_sum(sq) / static_cast<float>(N) + eps);
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int n = lane + 64 * i;
-    if (n < N) ln_out[base + n] = (v[i] - mean) * inv * g[n] + b[n];
-  }
-}
-
-template <int BM, int BN, int WGM, int WGN, int MINW, bool VEC>
-int launch_sg(SgemmArgs a, int batch, int splits, hipStream_t s) {
-  a.k_split = a.K;
-  a.part = nullptr;
-  if (splits > 1) {
-    a.k_split = ((a.K + splits - 1) / splits + kSK - 1) / kSK * kSK;
-    splits = (a.K + a.k_split - 1) / a.k_split;
-  }
-  a.batch = batch;
-  a.splits = splits;
-  const long MN = static_cast<long>(a.M) * a.N;
-  if (splits > 1) {
-    a.part = static_cast<float*>(
-        workspace(s, static_cast<size_t>(splits) * batch * MN * sizeof(float), kWsGemm));
-    if (!a.part) return ORATOR_ERR_HIP;
-  }
-  const dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, batch * splits);
-  const dim3 block(64 * WGM * WGN);
-  if (splits > 1)
-    hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WGM, WGN, MINW, VEC, kSEpiPartial>), grid, block,
-                       0, s, a);
-  else if (a.bias || a.act || a.residual || a.group)
-    hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WGM, WGN, MINW, VEC, kSEpiAct>), grid, block, 0,
-                       s, a);
-  else
-    hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WGM, WGN, MINW, VEC, kSEpiStore>), grid, block,
-                       0, s, a);
-  if (int rc = check_launch("sgemm_nt_kernel")) return rc;
-  if (splits == 1) {
-    if (!a.ln_g) return ORATOR_OK;
-    return launch_layer_norm(a.out, a.ln_g, a.ln_b, a.ln_out, a.M, a.N, a.ln_eps, s);
-  }
-  if (a.ln_g && a.N <= 1024 && splits <= kMaxLnSplits) {  // batch 1, act 0, residual
-    const dim3 rgrid((a.M + 3) / 4);
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, rgrid, dim3(256), 0, s, a.part, splits, a.bias, a.out, a.M, a.N,
-                         a.res_scale, a.ln_g, a.ln_b, a.ln_out, a.ln_eps);
-    };
-    if (a.N <= 512)
-      splits <= 2 ? go(sgemm_splitk_reduce_ln_kernel<8, 2>) : go(sgemm_splitk_reduce_ln_kernel<8, 8>);
-    else
-      splits <= 2 ? go(sgemm_splitk_reduce_ln_kernel<16, 2>) : go(sgemm_splitk_reduce_ln_kernel<16, 8>);
-    return check_launch("sgemm_splitk_reduce_ln");
-  }
-  const long total = MN * batch;
-  hipLaunchKernelGGL(sgemm_splitk_reduce_kernel, dim3(static_cast<unsigned>((total + 255) / 256)),
-                     dim3(256), 0, s, a.part, splits, batch, a.bias, a.out, a.M, a.N, a.act,
-                     batch > 1 ? a.s_out : MN, a.residual, a.res_scale);
-  if (int rc = check_launch("sgemm_splitk_reduce")) return rc;
-  if (!a.ln_g) return ORATOR_OK;
-  return launch_layer_norm(a.out, a.ln_g, a.ln_b, a.ln_out, a.M, a.N, a.ln_eps, s);
-}
-
-// 64 x 64 tiles, 4 waves of one 32 x 32 block each, four workgroups per CU.  K is split over
-// workgroups only when the grid leaves more than half the CUs idle.  Measured at the
-// Conformer's shapes: 717 x 2048 -> 512 takes 25 us with 8 splits against 45.9 unsplit;
-// 1433 x 512 -> 512 (184 tiles) 13.6 unsplit against 19.1 with 2 splits.  Grouped products
-// are never split.  Two tiles on one CU are
-// MFMA-bound together (each takes twice as long), so an unsplit grid that would give some CUs
-// two 64 x 64 tiles takes 96 x 64 tiles (6 waves) when that needs fewer rounds of work and K
-// is long enough for the tiles to be MFMA-bound: 717 x 512 -> 2048 (384 tiles -> 256) 28.3 ->
-// 24.5 us, -> 1536 (288 -> 192) 27.5 -> 23.5 us; at K = 64 (8 x 717 x 64 -> 717) 96-row tiles
-// were slower, 16.1 against 12.9 us.
-int run_sgemm(SgemmArgs a, int batch, hipStream_t stream) {
-  const int M = a.M, N = a.N, K = a.K;
+// Tile and waves by K and grid.  Many small tiles keep every CU busy where the grid is short;
+// larger tiles split fewer elements per MFMA.  Eight waves per tile shorten a short grid's time
+// (126 x 512 -> 512: 5.8 us, 6.1 with four) and, for long K, keep the partial sums short (K =
+// 2048: error 1.7e-7, four waves 2.4e-7); four let two to five workgroups share a CU, so that
+// one's first loads and epilogue run under the others' MFMAs (717 x 512 -> 2048: 32 x 64 tiles,
+// four waves 17.5 us, eight 20.8; 2000 x 512 -> 2048: 64 x 64, four waves 34.6, eight 43.3, 32 x
+// 64 38.3; 717 x 512 -> 1536: 32 x 32, four waves 15.8, eight 17.3, 32 x 64 16.2; 717 x 2048 ->
+// 512: 32 x 64, eight waves 17.6, 32 x 32 20.0, 64 x 64 25.6).  Short K (few slices per tile): 32 x 32
+// tiles, bound by the outputs written (8 x (717 x 64 -> 717): two waves 14.1 us, 32 x 64 15.8,
+// 64 x 64 21.7).
+template <bool VEC, bool GLU>
+int launch_sized(const SgemmArgs& a, hipStream_t s) {
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const long t = static_cast<long>((M + 63) / 64) * ((N + 63) / 64) * batch;
-  int splits = 1;
-  if (2 * t <= cus && K >= 512 && !a.group && !a.h16) {
-    // the split count with the least work per CU in whole rounds, ceil(t s / cus) / s (ties to
-    // fewer splits), K / 256 and 8 at most: 717 x 2048 -> 512 (96 tiles) takes 8 splits (768
-    // workgroups, 3 rounds of 1/8): 24.7-25.9 us, against 25.9-27.4 with 5 and 27.5-28.9 with 6
-    long best_num = 1, best_den = 1;  // 1 round of the whole K
-    for (long sp = 2; sp <= std::min<long>(8, K / 256); ++sp) {
-      const long rounds = (t * sp + cus - 1) / cus;
-      if (rounds * best_den < best_num * sp) {
-        best_num = rounds;
-        best_den = sp;
-      }
-    }
-    splits = static_cast<int>(best_den);
+  auto tiles = [&](int bm, int bn) {
+    return static_cast<long>((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
+  };
+  if (a.K >= 1024) {
+    if (tiles(32, 32) <= cus) return launch_tile<32, 32, 8, VEC, GLU>(a, s);
+    if (tiles(32, 64) <= 2 * cus) return launch_tile<32, 64, 8, VEC, GLU>(a, s);
+    return launch_tile<64, 64, 8, VEC, GLU>(a, s);
   }
-  if (static_cast<long>(batch) * splits > 65535) splits = 1;
-  if (splits == 1 && t > cus && K >= 256) {  // short K: latency-bound tiles, more is better
-    const long t96 = static_cast<long>((M + 95) / 96) * ((N + 63) / 64) * batch;
-    const long r64 = (t + cus - 1) / cus, r96 = (t96 + cus - 1) / cus;
-    if (2 * r64 > 3 * r96) {  // rounds of 64 x 64 work: r64 against 1.5 r96
-      if (a.vec) return launch_sg<96, 64, 3, 2, 2, true>(a, batch, 1, stream);
-      return launch_sg<96, 64, 3, 2, 2, false>(a, batch, 1, stream);
-    }
+  if (a.K >= 256) {
+    if (2 * tiles(32, 32) <= 3 * cus) return launch_tile<32, 32, 8, VEC, GLU>(a, s);
+    if (tiles(32, 32) <= 5 * cus) return launch_tile<32, 32, 4, VEC, GLU>(a, s);
+    if (tiles(32, 64) <= 4 * cus) return launch_tile<32, 64, 4, VEC, GLU>(a, s);
+    return launch_tile<64, 64, 4, VEC, GLU>(a, s);
   }
-  if (a.vec) return launch_sg<64, 64, 2, 2, 4, true>(a, batch, splits, stream);
-  return launch_sg<64, 64, 2, 2, 4, false>(a, batch, splits, stream);
+  if (tiles(32, 32) <= 4 * cus) return launch_tile<32, 32, 4, VEC, GLU>(a, s);
+  return launch_tile<32, 32, 2, VEC, GLU>(a, s);
+}
+
+int run_sgemm(SgemmArgs a, int batch, bool glu, hipStream_t s) {
+  a.batch = batch;
+  a.chain = a.K >= (1 << 24);  // 64 rows of K floats past 4 GB
+  const int rc = glu ? launch_sized<true, true>(a, s)
+                 : a.vec ? launch_sized<true, false>(a, s) : launch_sized<false, false>(a, s);
+  if (rc || !a.ln_g) return rc;
+  return launch_layer_norm(a.out, a.ln_g, a.ln_b, a.ln_out, a.M, a.N, a.ln_eps, s);
 }
 
 }  // namespace
@@ -548,7 +462,7 @@ int launch_sgemm(const float* in, const float* W, const float* bias, float* out,
   a.s_out = batch > 1 ? stride_out : 0;
   a.vec = (K % kSK) == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W) |
                             (batch > 1 ? (stride_in | stride_w) * 4 : 0)) & 15) == 0;
-  return run_sgemm(a, batch, stream);
+  return run_sgemm(a, batch, false, stream);
 }
 
 int launch_sgemm_residual(const float* in, const float* W, const float* bias, float* out, int M,
@@ -567,7 +481,7 @@ int launch_sgemm_residual(const float* in, const float* W, const float* bias, fl
   a.res_scale = res_scale;
   a.vec = (K % kSK) == 0 &&
           ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  return run_sgemm(a, 1, stream);
+  return run_sgemm(a, 1, false, stream);
 }
 
 int launch_sgemm_residual_ln(const float* in, const float* W, const float* bias, float* out,
@@ -592,7 +506,7 @@ int launch_sgemm_residual_ln(const float* in, const float* W, const float* bias,
   a.ln_eps = eps;
   a.vec = (K % kSK) == 0 &&
           ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  return run_sgemm(a, 1, stream);
+  return run_sgemm(a, 1, false, stream);
 }
 
 int launch_sgemm_glu(const float* in, const float* W, const float* bias, float* out, int M, int K,
@@ -610,16 +524,10 @@ int launch_sgemm_glu(const float* in, const float* W, const float* bias, float* 
   a.M = M;
   a.K = K;
   a.N = 2 * C;
-  a.k_split = K;
-  a.batch = 1;
-  a.splits = 1;
   a.vec = true;
   a.glu_c = C;
   a.glu_valid = valid;
-  const dim3 grid((C + 31) / 32, (M + 63) / 64, 1);
-  hipLaunchKernelGGL((sgemm_nt_kernel<64, 64, 2, 2, 4, true, kSEpiGlu>), grid, dim3(256), 0, stream,
-                     a);
-  return check_launch("sgemm_nt_kernel (glu)");
+  return run_sgemm(a, 1, true, stream);
 }
 
 int launch_sgemm_group3(const float* in, const float* const W[3], const float* const bias[3],
@@ -644,7 +552,7 @@ int launch_sgemm_group3(const float* in, const float* const W[3], const float* c
   }
   a.W = a.Wg[0];
   a.vec = (K % kSK) == 0 && (align & 15) == 0;
-  return run_sgemm(a, 3, stream);
+  return run_sgemm(a, 3, false, stream);
 }
 
 int launch_sgemm_f16_out(const float* in, const float* W, void* out, int M, int K, int N,
@@ -661,7 +569,7 @@ int launch_sgemm_f16_out(const float* in, const float* W, void* out, int M, int 
   a.h16 = 1;
   a.vec = (K % kSK) == 0 &&
           ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  return run_sgemm(a, 1, stream);
+  return run_sgemm(a, 1, false, stream);
 }
 
 }  // namespace orator_hip
