@@ -7,6 +7,9 @@
 // consecutive k per lane), so tiles go from HBM to LDS row by row and back out as fragments
 // without any transpose.
 //
+// This register-staged kernel serves what gemm_dma.hip's does not take: K not a multiple of 64, N not
+// of 4, unaligned operands, sizes past 32-bit offsets.
+//
 // Workgroup = BM x BN output tile, 4 waves (one per SIMD) in a WGM x WGN grid, each wave
 // (BM/WGM) x (BN/WGN) = FM x FN blocks of 32 x 32 accumulators, two workgroups per CU (73.7 KB
 // of LDS each), so one workgroup's epilogue and barrier waits overlap the other's MFMAs.  K
@@ -380,9 +383,11 @@ int launch_tile(const uint16_t* in, const uint16_t* W, const float* bias, float*
 int launch_gemm_bf16_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out, float* tmp,
                             int M, int K, int I, hipStream_t s) {
   if (M <= 0 || K <= 0 || I <= 0) return ORATOR_OK;
+  const bool dma = I % 4 == 0 && gemm_dma_takes(in, W, out, M, K, 2 * I);
+  if (dma && !gemm_dma_splits(M, K, 2 * I)) return launch_gemm_dma_swiglu(in, W, out, M, K, I, s);
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const long tiles = static_cast<long>((M + 127) / 128) * ((I + 63) / 64);
-  if (tiles < cus) {
+  if (dma || tiles < cus) {
     if (!tmp) tmp = static_cast<float*>(workspace(s, static_cast<size_t>(M) * 2 * I * sizeof(float)));
     if (!tmp) return ORATOR_ERR_HIP;
     if (int rc = launch_gemm_bf16_nt(in, W, nullptr, tmp, M, K, 2 * I, 0, false, s)) return rc;
@@ -404,6 +409,8 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic) {
   if (M <= 0 || K <= 0 || N <= 0) return ORATOR_OK;
+  if (!generic && gemm_dma_takes(in, W, out, M, K, N))
+    return launch_gemm_dma(in, W, bias, out, M, K, N, act, accumulate, s);
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   auto tiles = [&](int bm, int bn) {
     return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);

@@ -182,6 +182,16 @@ int launch_swiglu_bf16(const float* gu, uint16_t* out, int T, int I, hipStream_t
 int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias, float* out,
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic = false);
+// The same on tiles loaded straight into LDS (gemm_dma.hip), for the operands gemm_dma_takes: K a
+// multiple of 64, N of 4, 16-byte aligned pointers, 32-bit sizes.  SwiGLU: N = 2I, I a multiple of 4.
+bool gemm_dma_takes(const void* in, const void* W, const void* out, int M, int K, int N);
+int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, float* out, int M,
+                    int K, int N, int act, bool accumulate, hipStream_t s);
+// Whether launch_gemm_dma splits K for this shape: its sums are then in another order than the
+// unsplit SwiGLU form's.
+bool gemm_dma_splits(int M, int K, int N);
+int launch_gemm_dma_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out, int M, int K,
+                           int I, hipStream_t s);
 // The gate|up projection with SwiGLU and the bf16 cast in the GEMM epilogue (gemm_bf16.hip):
 // out[M][I] = bf16(silu(in W[0:I]^T) * (in W[I:2I]^T)); `tmp` ([M][2I] fp32, or null for the
 // stream's workspace) is used only when the grid is too short for the fused kernel.

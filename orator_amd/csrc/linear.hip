@@ -9,7 +9,7 @@
 //    4 output rows; each lane reads 16 contiguous bytes of each row per step, so a wave
 //    instruction moves one contiguous 1 KB piece of a row, and the k loop is unrolled so a
 //    lane keeps 16 such loads in flight.  x (4-12 KB) is read through the caches.
-//  * M > 1 (prefill) is MFMA-bound: this library's bf16 GEMM (gemm_bf16.hip).
+//  * M > 1 (prefill) is MFMA-bound: this library's bf16 GEMM (gemm_dma.hip, gemm_bf16.hip).
 //  * K not a multiple of 8, or operands not 16-byte aligned (the audio tower's first conv as
 //    a GEMM has K = 9, asr_audio_tower.cu:417-445): the GEMM with element loads, M = 1 too.
 #include "common.hpp"

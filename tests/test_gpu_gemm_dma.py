@@ -1,0 +1,55 @@
+"""GPU: the bf16 GEMM on tiles loaded straight into LDS (gemm_dma.hip) at the edges of its tiles,
+stages, K splits and dispatch.  Operands are small integers (exact in bf16) and every sum stays
+below 2^24, so any order of fp32 additions gives the exact integer: equality, no tolerance."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+from gpu_helpers import down, empty, say, up
+from orator_amd import asr_gemm, asr_ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _ints(r, shape, lim):
+    return r.integers(-lim, lim + 1, shape).astype(np.float32)
+
+
+# 64 x 64 tiles: one row pair, ragged rows and columns, one K step, fewer steps than stages, uneven K
+# splits; 128 x 128 with 4 stages (one tile per CU at most); 128 x 128 with 2; 256 x 192; K not a
+# multiple of 64 and N not of 4 (the register-staged kernel) beside them
+@pytest.mark.parametrize("M,K,N", [(2, 64, 4), (63, 128, 60), (65, 192, 68), (130, 320, 516),
+                                   (3, 2048, 2044), (65, 4160, 1000), (503, 4160, 2048),
+                                   (2000, 64, 2044), (1921, 320, 2044), (2000, 64, 4092),
+                                   (1921, 192, 4036), (2040, 64, 12284), (1793, 192, 12100),
+                                   (130, 72, 516), (130, 64, 514)])
+@pytest.mark.parametrize("bias,act", [(False, 0), (True, 2)])
+def test_gemm_dma_exact(M, K, N, bias, act):
+    r = np.random.default_rng(M + K + N)
+    x, w, b = _ints(r, (M, K), 4), _ints(r, (N, K), 4), _ints(r, (N,), 100)
+    out = empty((M, N), np.float32)
+    say("gemm dma", M, K, N, bias, act)
+    asr_gemm.LinearPre(up(orc.to_bf16(x)), up(orc.to_bf16(w)), up(b) if bias else None, out, M, K, N,
+                       act)
+    ref = x @ w.T + (b if bias else 0)
+    np.testing.assert_array_equal(down(out, (M, N)), np.maximum(ref, 0) if act == 2 else ref)
+
+
+@pytest.mark.parametrize("M,K,I", [(2, 64, 4), (65, 192, 100), (17, 2048, 64), (503, 128, 6140),
+                                   (1921, 64, 1024), (2040, 192, 6140)])
+def test_gemm_dma_swiglu_bits(M, K, I):
+    """The same bits as LinearPre, SwiGLU and the cast, on every tile and where K is split."""
+    r = np.random.default_rng(M + K + I)
+    x = up(orc.to_bf16(r.standard_normal((M, K)).astype(np.float32)))
+    w = up(orc.to_bf16((r.standard_normal((2 * I, K)) * K ** -0.5).astype(np.float32)))
+    gu, got = empty((M, 2 * I), np.float32), empty((M, I), np.uint16)
+    say("gemm dma swiglu", M, K, I)
+    asr_gemm.LinearPreSwiGLU(x, w, got, M, K, I)
+    asr_gemm.LinearPre(x, w, None, gu, M, K, 2 * I, 0)
+    g = down(gu, (M, 2 * I))
+    act, want = empty((M, I), np.float32), empty((M, I), np.uint16)
+    asr_ops.SwiGLU(up(np.ascontiguousarray(g[:, :I])), up(np.ascontiguousarray(g[:, I:])), act, M * I)
+    asr_ops.F32ToBf16(act, want, M * I)
+    np.testing.assert_array_equal(down(got, (M, I), np.uint16), down(want, (M, I), np.uint16))
