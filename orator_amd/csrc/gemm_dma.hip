@@ -28,10 +28,12 @@
 namespace orator_hip {
 namespace {
 
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 enum GemmEpi : int { kDmaStore = 0, kDmaPartial = 1, kDmaAct = 2, kDmaSwiglu = 3 };
 
 struct GemmDmaArgs {
-  const uint16_t* A;
+  const void* A;  // bf16, or fp32 (the F32 kernels)
   const uint16_t* W;
   const float* bias;
   void* out;    // fp32 [M][N]; SwiGLU: bf16 [M][N / 2]
@@ -45,17 +47,29 @@ __device__ __forceinline__ float gemm_act(float v, int act) {
   return v;
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, int MINW, int EPI>
+// Eight fp32 values as bf16 (v_cvt_pk_bf16_f32: to nearest even, as the cast kernel; a NaN stays one
+// whatever its payload).
+__device__ __forceinline__ bf16x8_t cvt_bf16x8(const f32x4_t lo, const f32x4_t hi) {
+  return as_bf16x8(make_uint4(cvt_bf16x2(lo[0], lo[1]), cvt_bf16x2(lo[2], lo[3]),
+                              cvt_bf16x2(hi[0], hi[1]), cvt_bf16x2(hi[2], hi[3])));
+}
+
+// F32: A is fp32 and lies in LDS as such, 256-byte rows with chunk c at c ^ r % 16; it is rounded as
+// the fragments are read.
+template <int BM, int BN, int WGM, int WGN, int NS, int MINW, int EPI, bool F32>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(GemmDmaArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass has no LDS loads; it needs the launch stub only
   constexpr int BK = 64, CH = BK / 8;          // 16-byte chunks per tile row
   constexpr int NW = WGM * WGN;
   constexpr int TM = BM / WGM, TN = BN / WGN;  // wave tile
   constexpr int FM = TM / 32, FN = TN / 32;
-  constexpr int RPI = 64 / CH;                 // tile rows per load instruction of a wave
-  constexpr int L = (BM + BN) / RPI / NW;      // load instructions per wave and stage
-  static_assert((BM + BN) % (RPI * NW) == 0 && TM % 32 == 0 && TN % 32 == 0 && NS >= 2 && NS <= 4);
-  constexpr int kStage = (BM + BN) * BK;
+  constexpr int CHA = F32 ? 2 * CH : CH;       // the same of an A row
+  constexpr int RPA = 64 / CHA, RPW = 64 / CH;  // tile rows per load instruction of a wave
+  constexpr int LA = BM / RPA;                 // load instructions of the A tile
+  constexpr int L = (LA + BN / RPW) / NW;      // load instructions per wave and stage
+  static_assert(LA % NW == 0 && BN / RPW % NW == 0 && BM % RPA == 0 && BN % RPW == 0 && TM % 32 == 0 && TN % 32 == 0 && NS >= 2 && NS <= 4);
+  constexpr int kA = BM * CHA * 8;             // the A tile's part of a stage, in 2-byte units
+  constexpr int kStage = kA + BN * BK;
   // One array per stage: the compiler's own waits before an LDS read then count the loads into
   // that stage only, and the later stages' loads stay in flight.
   __shared__ __align__(1024) uint16_t s0[kStage], s1[kStage];
@@ -78,8 +92,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   const int M = a.M, N = a.N, K = a.K;
   const int kb = blockIdx.z * a.k_split;
   const int n_k = min(K - kb, a.k_split) / BK;
-  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.A), 0,
-                                                      static_cast<uint32_t>(M) * K * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.A), 0,
+                                                      static_cast<uint32_t>(M) * K * (F32 ? 4 : 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.W), 0,
                                                       static_cast<uint32_t>(N) * K * 2, 0x00020000);
   // W row of tile row j
@@ -95,18 +109,27 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   uint32_t voff[L];
 #pragma unroll
   for (int i = 0; i < L; ++i) {
-    const int r = (wave + NW * i) * RPI + lane / CH;
-    const int row = r < BM ? min(m0 + r, M - 1) : w_row(r - BM);
-    voff[i] = static_cast<uint32_t>(row) * K * 2 + 16 * ((lane % CH) ^ swz(r)) + kb * 2;
+    const int ins = wave + NW * i;
+    if (i < LA / NW) {
+      const int r = ins * RPA + lane / CHA;
+      const int chunk = (lane % CHA) ^ (F32 ? r & (CHA - 1) : swz(r));
+      voff[i] = (static_cast<uint32_t>(min(m0 + r, M - 1)) * K + kb) * (F32 ? 4 : 2) + 16 * chunk;
+    } else {
+      const int r = (ins - LA) * RPW + lane / CH;
+      voff[i] = (static_cast<uint32_t>(w_row(r)) * K + kb) * 2 + 16 * ((lane % CH) ^ swz(r));
+    }
   }
   auto issue = [&](uint16_t* st, int t) {
 #pragma unroll
     for (int i = 0; i < L; ++i) {
       const int ins = wave + NW * i;
-      const __amdgpu_buffer_rsrc_t rs = ins < BM / RPI ? rs_a : rs_w;
+      const bool is_a = i < LA / NW;  // known at compile time: a branch here or in the addresses
+      // above costs the stages' separation (the compiler then waits for every load in flight)
+      const __amdgpu_buffer_rsrc_t rs = is_a ? rs_a : rs_w;
+      // every load instruction fills 1024 bytes (512 units), A's first
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs, (__attribute__((address_space(3))) void*)(st + ins * RPI * BK), 16, voff[i],
-          t * (BK * 2), 0, 0);
+          rs, (__attribute__((address_space(3))) void*)(st + ins * 512), 16, voff[i],
+          t * (F32 && is_a ? BK * 4 : BK * 2), 0, 0);
     }
   };
 
@@ -121,17 +144,26 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   const int fx = swz(fr);
 
   auto compute = [&](const uint16_t* st) {
-    const uint16_t* pa = st + (wm * TM + fr) * BK;
-    const uint16_t* pw = st + (BM + wn * TN + fr) * BK;
+    const uint16_t* pa = st + (wm * TM + fr) * (kA / BM);
+    const uint16_t* pw = st + (kA / BK + wn * TN + fr) * BK;
     bf16x8_t fa[2][FM], fb[2][FN];
+    [[maybe_unused]] f32x4_t ra[2][FM][2];
     auto read = [&](int ks, int s) {
       const int c = 8 * ((2 * ks + hi) ^ fx);
 #pragma unroll
       for (int j = 0; j < FN; ++j)
         fb[s][j] = *reinterpret_cast<const bf16x8_t*>(pw + 32 * j * BK + c);
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-        fa[s][i] = *reinterpret_cast<const bf16x8_t*>(pa + 32 * i * BK + c);
+      for (int i = 0; i < FM; ++i) {
+        if constexpr (F32) {
+          const uint16_t* row = pa + 32 * i * (kA / BM);
+          const int c2 = 4 * ks + 2 * hi, x = fr & (CHA - 1);
+          ra[s][i][0] = *reinterpret_cast<const f32x4_t*>(row + 8 * (c2 ^ x));
+          ra[s][i][1] = *reinterpret_cast<const f32x4_t*>(row + 8 * ((c2 + 1) ^ x));
+        } else {
+          fa[s][i] = *reinterpret_cast<const bf16x8_t*>(pa + 32 * i * BK + c);
+        }
+      }
     };
     read(0, 0);
 #pragma unroll
@@ -139,6 +171,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
       const int s = ks & 1;
       if (ks + 1 < BK / 16) read(ks + 1, s ^ 1);
       __builtin_amdgcn_sched_barrier(0);  // the next fragments are on their way under these MFMAs
+      if constexpr (F32) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) fa[s][i] = cvt_bf16x8(ra[s][i][0], ra[s][i][1]);
+      }
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -251,7 +287,7 @@ __global__ __launch_bounds__(256) void gemm_dma_reduce_kernel(GemmDmaArgs a, int
   *dst = v;
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, int MINW, bool SWIGLU>
+template <int BM, int BN, int WGM, int WGN, int NS, int MINW, bool SWIGLU, bool F32 = false>
 int launch_tile(GemmDmaArgs a, int splits, hipStream_t s) {
   const int steps = a.K / 64;
   const int per = (steps + splits - 1) / splits;
@@ -259,7 +295,7 @@ int launch_tile(GemmDmaArgs a, int splits, hipStream_t s) {
   a.k_split = 64 * per;
   const dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, splits), block(64 * WGM * WGN);
   if constexpr (SWIGLU) {
-    hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaSwiglu>), grid, block,
+    hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaSwiglu, F32>), grid, block,
                        0, s, a);
     return check_launch("gemm_bf16_dma_kernel (swiglu)");
   } else {
@@ -267,7 +303,7 @@ int launch_tile(GemmDmaArgs a, int splits, hipStream_t s) {
       const size_t bytes = static_cast<size_t>(splits) * a.M * a.N * sizeof(float);
       a.part = static_cast<float*>(workspace(s, bytes, kWsGemm));
       if (!a.part) return ORATOR_ERR_HIP;
-      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaPartial>), grid,
+      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaPartial, F32>), grid,
                          block, 0, s, a);
       if (int rc = check_launch("gemm_bf16_dma_kernel")) return rc;
       const unsigned quads = static_cast<unsigned>(static_cast<long>(a.M) * a.N / 4);
@@ -276,10 +312,10 @@ int launch_tile(GemmDmaArgs a, int splits, hipStream_t s) {
       return check_launch("gemm_dma_reduce_kernel");
     }
     if (a.bias || a.act || a.accumulate)
-      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaAct>), grid, block,
+      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaAct, F32>), grid, block,
                          0, s, a);
     else
-      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaStore>), grid, block,
+      hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WGM, WGN, NS, MINW, kDmaStore, F32>), grid, block,
                          0, s, a);
     return check_launch("gemm_bf16_dma_kernel");
   }
@@ -314,13 +350,17 @@ Shape pick_shape(int M, int K, int N) {
   const double c64 = cost(t64, 2 * cus, 14.4, 11.3);
   if (c256 < c128 && c256 < c64) return {Tile::k256x192, 1};
   if (c128 < c64) return {t128 <= cus ? Tile::k128x128Deep : Tile::k128x128, 1};
-  // A grid of at most half the CUs, or one workgroup per CU over a long K: split K until the chip
-  // has two per CU, 512 of K at least each (the reduction is a launch of 4 us: 503 x 6144 -> 2048
-  // 31.8 unsplit, 23.4 + 4 split; 503 x 2048 -> 2048 11.3 unsplit, 10.1 + 4 split).
-  int splits = 1;
-  if (2 * t64 <= cus || (t64 <= cus && K >= 4096))
-    splits = static_cast<int>(std::min<long>((2 * cus + t64 - 1) / t64, std::max(1, K / 512)));
-  return {Tile::k64x64, splits};
+  // A grid of at most half the CUs: K split until every CU has a workgroup, 512 of K each at least, or
+  // two, 1024 each (us: 100 x 2048 -> 2048 10.1 unsplit, 5.0 and a reduction of 4 split by 4; 200 x
+  // 2048 -> 2048 13.8 by 2, 14.5 by 4; 200 x 6144 -> 2048 24.3 by 2, 21.2 by 4).  One workgroup per CU
+  // over a long K: split by two (503 x 6144 -> 2048 31.8 unsplit, 23.4 + 4; 503 x 2048 -> 2048, 11.3
+  // and 10.1 + 4, stays whole; a third part would start another round: 390 x 6144 -> 2048 3 us slower).
+  long splits = 1;
+  if (2 * t64 <= cus)
+    splits = std::max({std::min<long>(cus / t64, K / 512), std::min<long>(2 * cus / t64, K / 1024), 1L});
+  else if (t64 <= cus && K >= 4096)
+    splits = 2;
+  return {Tile::k64x64, static_cast<int>(splits)};
 }
 
 template <bool SWIGLU>
@@ -352,6 +392,25 @@ int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, fl
                     int K, int N, int act, bool accumulate, hipStream_t s) {
   return launch_shape<false>(
       GemmDmaArgs{in, W, bias, out, nullptr, M, K, N, act, accumulate ? 1 : 0, K}, s);
+}
+
+// fp32 activations of up to 128 rows: the cast pass is a launch and a round trip through memory, which
+// the fused form saves (us with cold operands, cast + GEMM against fused: 2048 -> 2048 15.3 and 12.8
+// at 2 rows, 16.9 and 14.4 at 128; 1024 -> 4096 17.1 and 14.6 at 128).  The A tile takes twice the LDS
+// bandwidth and two of three stages' room, so with more rows the pass is cheaper (2048 -> 4096 at 200
+// rows 24.0 and 26.3, at 512 30.6 and 34.0; 6144 -> 2048 at 200 29.1 and 34.0).
+bool gemm_dma_takes_f32(const float* in, const void* W, const float* out, int M, int K, int N) {
+  const uintptr_t ib = reinterpret_cast<uintptr_t>(in), ob = reinterpret_cast<uintptr_t>(out);
+  const bool apart = ib + 4 * static_cast<uintptr_t>(M) * K <= ob ||
+                     ob + 4 * static_cast<uintptr_t>(M) * N <= ib;
+  return M > 1 && M <= 128 && apart && gemm_dma_takes(in, W, out, M, K, N) && fits32(M, 2 * K, N) &&
+         pick_shape(M, K, N).tile == Tile::k64x64;
+}
+
+int launch_gemm_dma_f32(const float* in, const uint16_t* W, const float* bias, float* out, int M,
+                        int K, int N, int act, hipStream_t s) {
+  return launch_tile<64, 64, 2, 2, 3, 2, false, true>(
+      GemmDmaArgs{in, W, bias, out, nullptr, M, K, N, act, 0, K}, pick_shape(M, K, N).splits, s);
 }
 
 bool gemm_dma_splits(int M, int K, int N) { return pick_shape(M, K, N).splits > 1; }

@@ -187,6 +187,10 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
 bool gemm_dma_takes(const void* in, const void* W, const void* out, int M, int K, int N);
 int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, float* out, int M,
                     int K, int N, int act, bool accumulate, hipStream_t s);
+// The same from fp32 activations, rounded to bf16 inside the kernel; `out` apart from `in`.
+bool gemm_dma_takes_f32(const float* in, const void* W, const float* out, int M, int K, int N);
+int launch_gemm_dma_f32(const float* in, const uint16_t* W, const float* bias, float* out, int M,
+                        int K, int N, int act, hipStream_t s);
 // Whether launch_gemm_dma splits K for this shape: its sums are then in another order than the
 // unsplit SwiGLU form's.
 bool gemm_dma_splits(int M, int K, int N);

@@ -415,6 +415,8 @@ int orator_linear(const float* in_f32, const uint16_t* W_bf16, const float* bias
   if (M <= 0 || K <= 0 || N <= 0) return ORATOR_OK;
   if (!in_f32) return fail(ORATOR_ERR_INVALID, "linear: null pointer");
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (W_bf16 && out && act >= 0 && act <= 2 && gemm_dma_takes_f32(in_f32, W_bf16, out, M, K, N))
+    return launch_gemm_dma_f32(in_f32, W_bf16, bias, out, M, K, N, act, s);
   const long n = static_cast<long>(M) * K;
   uint16_t* in_bf16 = static_cast<uint16_t*>(workspace(s, n * sizeof(uint16_t)));
   if (!in_bf16) return ORATOR_ERR_HIP;

@@ -53,3 +53,36 @@ def test_gemm_dma_swiglu_bits(M, K, I):
     asr_ops.SwiGLU(up(np.ascontiguousarray(g[:, :I])), up(np.ascontiguousarray(g[:, I:])), act, M * I)
     asr_ops.F32ToBf16(act, want, M * I)
     np.testing.assert_array_equal(down(got, (M, I), np.uint16), down(want, (M, I), np.uint16))
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 64, 4), (63, 128, 60), (65, 192, 68), (130, 320, 516),
+                                   (3, 2048, 2044), (65, 4160, 1000), (128, 1024, 4096), (129, 1024, 4096),
+                                   (1921, 320, 2044), (130, 72, 516)])
+def test_linear_rounds_like_the_cast(M, K, N):
+    """fp32 activations rounded inside the GEMM: the bits of F32ToBf16 + LinearPre, ties and both
+    infinities among the values."""
+    r = np.random.default_rng(M + K + N)
+    x = r.standard_normal((M, K)).astype(np.float32)
+    tie = r.integers(0, K, M)
+    x[np.arange(M), tie] = np.float32(1 + 2.0 ** -8) * r.choice([1, -1, 3], M)
+    x[0, 0], x[1, K - 1] = np.inf, -np.inf
+    w = up(orc.to_bf16((r.standard_normal((N, K)) * K ** -0.5).astype(np.float32)))
+    a, b = empty((M, N), np.float32), empty((M, N), np.float32)
+    bias = up(r.standard_normal(N).astype(np.float32))
+    say("linear f32", M, K, N)
+    asr_gemm.Linear(up(x), w, bias, a, M, K, N, 1)
+    xb = empty((M, K), np.uint16)
+    asr_ops.F32ToBf16(up(x), xb, M * K)
+    asr_gemm.LinearPre(xb, w, bias, b, M, K, N, 1)
+    np.testing.assert_array_equal(down(a, (M, N)), down(b, (M, N)))
+
+
+def test_linear_in_place():
+    """Output over the input (K = N): through the cast copy, as before."""
+    r = np.random.default_rng(9)
+    M, K = 70, 256
+    x, w = _ints(r, (M, K), 4), _ints(r, (K, K), 4)
+    buf = up(x)
+    say("linear in place")
+    asr_gemm.Linear(buf, up(orc.to_bf16(w)), None, buf, M, K, K, 0)
+    np.testing.assert_array_equal(down(buf, (M, K)), x @ w.T)
