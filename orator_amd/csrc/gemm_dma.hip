@@ -2,8 +2,7 @@
 // out[M][N] (=|+=) act(in[M][K] W[N][K]^T + bias), and the gate|up form with SwiGLU.
 //
 // Serves every M > 1 product of gemm_bf16.hip's entry points whose K is a multiple of 64 (all of
-// the decoder's and the audio tower's); the values are those of the register-staged kernel there,
-// bit for bit (same MFMA, same order of k).
+// the decoder's and the audio tower's).
 //
 // What bounds it: the matrix cores and LDS bandwidth at once.  A 64 x 64 wave tile reads LDS as
 // long as its MFMAs run (4 KB and 4 MFMAs of 32 cycles per 16 of K, 128 bytes a cycle for 4 waves),
@@ -11,7 +10,10 @@
 //  * Buffer loads with an LDS destination: no staging registers and no ds_write.  The register-
 //    staged kernel ran at 760 TFLOP/s on 2048 x 2048 -> 12288, this one at 1118 (135.6 -> 92.2 us).
 //  * NS stages with one barrier per 64 of K; NS - 1 stages are in flight, which is what cold
-//    weights need (390 x 1024 -> 4096 from HBM: 20.0 -> 14.7 us).
+//    weights need (390 x 1024 -> 4096 from HBM: 20.0 -> 14.7 us).  Loads past the last stage are
+//    issued all the same (its tile again): with a branch around them the compiler cannot count what
+//    is in flight and waits for all of it at some stages (2048 x 6144 -> 2048, 1500 rows: 53.4 ->
+//    44.3 us; 200 x 2048 -> 12288 21.3 -> 17.7).
 //  * Rows of 128 bytes, unpadded (a load writes consecutive LDS bytes); the 16-byte chunk c of row r
 //    lies at c ^ (r / 2) % 8, so the 16 rows a quarter-wave reads cover all banks once.  The
 //    permutation is applied to the addresses the lanes load from.
@@ -133,13 +135,19 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
     }
   };
 
-  f32x16_t acc[FM][FN];
+  // One block per wave: the four k-steps of a stage add up apart, which shortens every chain of fp32
+  // additions to a quarter of K (the sums are then no further from 64 bits than K split
+  // by four left them).
+  constexpr int NA = FM * FN == 1 ? BK / 16 : 1;
+  f32x16_t part_acc[NA][FM][FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int h = 0; h < NA; ++h)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) part_acc[h][i][j][e] = 0.0f;
   const int fr = lane & 31, hi = lane >> 5;
   const int fx = swz(fr);
 
@@ -178,16 +186,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(fb[s][j], fa[s][i], acc[i][j]);
+        for (int j = 0; j < FN; ++j) part_acc[ks % NA][i][j] = mfma32(fb[s][j], fa[s][i], part_acc[ks % NA][i][j]);
     }
   };
-  auto ready = [&](int t) {  // stage t has arrived for every wave, stage t - 1 is read out
+  auto ready = [&] {  // stage t has arrived for every wave, stage t - 1 is read out
     // builtins, not asm: the compiler then knows what has arrived and adds no wait of its own
     constexpr int kLater = (NS - 2) * L;  // vmcnt bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8
-    if (t + NS - 2 < n_k)
-      __builtin_amdgcn_s_waitcnt(0x0070 | (kLater & 15) | (kLater >> 4) << 14);
-    else
-      __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_waitcnt(0x0070 | (kLater & 15) | (kLater >> 4) << 14);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -198,18 +203,24 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   };
 #pragma unroll
   for (int i = 0; i < NS - 1; ++i)
-    if (i < n_k) issue(stage(i), i);
+    issue(stage(i), min(i, n_k - 1));  // unconditional (a branch costs a wait for every load in flight)
   for (int t = 0; t < n_k; t += NS) {
 #pragma unroll
     for (int u = 0; u < NS; ++u) {
       if (t + u < n_k) {
-        ready(t + u);
-        if (t + u + NS - 1 < n_k) issue(stage(u + NS - 1), t + u + NS - 1);
+        ready();
+        issue(stage(u + NS - 1), min(t + u + NS - 1, n_k - 1));
         compute(stage(u));
       }
     }
   }
 
+  __builtin_amdgcn_s_waitcnt(0x0070);  // LDS is given back only when nothing is on its way to it
+  auto& acc = part_acc[0];
+#pragma unroll
+  for (int h = 1; h < NA; h *= 2)
+#pragma unroll
+    for (int g = 0; g + h < NA; g += 2 * h) part_acc[g][0][0] += part_acc[g + h][0][0];
   // Lane: output row fr of each block row, columns 8 (e / 4) + 4 hi + e % 4 of each block column.
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
