@@ -5,12 +5,19 @@
 // 2 ReLU, 3 sigmoid (gemm.cuh:38-45), strided batches, arbitrary M/N/K and alignment.
 //
 // fp32 products on the bf16 matrix cores: every operand is split in registers into three bf16
-// terms whose sum is the fp32 value exactly, and the six products of terms that reach fp32's
-// precision are accumulated in fp32 (what is dropped is below 2^-26 of |x w|, and the MFMA adds
-// 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96 cycles
+// terms, whose sum is the fp32 value exactly from 2^-103 on, and the six products of terms that
+// reach fp32's precision are accumulated in fp32 (what is dropped is below 2^-24 of |x w|, and the
+// MFMA adds 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96 cycles
 // per 16 x 16 x 32 block, the fp32 MFMA's 256.  Measured against 64 bits (random normal
 // operands, relative 2-norm): K = 512 0.8-1.2e-7, K = 2048 1.7e-7, K = 64 4.7e-8; the fp32 MFMA
 // 2.9e-7 unsplit (2.1e-7 with K in two parts), 2.1e-7 in eight parts, 1.4e-7.
+//
+// Results that the terms cannot carry are formed again by the wave on the fp32 MFMA: those that are
+// not finite, those so small that operands below 2^-103 may show in them, and all after an operand
+// of 2^32 or more.  One more MFMA per fragment finds the large operands (2-4 % of the time; a
+// class test of every element's third remainder found the small ones directly and took 12-25 %).
+// 717 x 512 -> 2048: 24 us with a NaN in one row, 19 with every second row zero, 36 with every
+// operand near 2^-118, against 26, 24 and 26 when every product was formed on the fp32 MFMA.
 //
 // Workgroup = BM x BN tile of one batch entry; its WK waves share the tile and split K: wave w
 // takes the 32-float slices w, w + WK, ..., accumulates the whole tile in registers, and the WK
@@ -30,7 +37,7 @@
 //   717 x 512 -> 2048  28.7 -> 16.3   717 x 2048 -> 512  24.5 -> 17.3   717 x 512 -> 512 12.2 -> 8.2
 //   717 x 512 -> 1536  27.0 -> 15.1   1433 x 512 -> 512  15.4 -> 10.6   717 x 512 -> 1024 15.4 -> 10.8
 //   126 x 512 -> 2048  11.2 -> 5.9    126 x 2048 -> 512  12.7 -> 11.9   126 x 512 -> 512 10.3 -> 5.8
-//   8 x (717 x 717 -> 64) 19.8 -> 13.5; 8 x (717 x 64 -> 717) 14.2 -> 14.1, 8 x (1000 x 64 -> 1999)
+//   8 x (717 x 717 -> 64) 19.8 -> 14.1; 8 x (717 x 64 -> 717) 14.2 -> 14.1, 8 x (1000 x 64 -> 1999)
 //   31.2 -> 36.6 (bound by its 64 MB of unaligned rows written).
 #include <stdint.h>
 
@@ -45,6 +52,7 @@ namespace orator_hip {
 namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kSK = 32;  // K per slice (floats)
 
@@ -83,14 +91,15 @@ struct SgemmArgs {
   const float* ln_b;
   float* ln_out;
   float ln_eps;
-  bool chain;  // every output as one fp32 chain (rows too long for 32-bit tile offsets)
   // fp16 outputs: bit z set stores problem z's output (group products; bit 0 otherwise) as
   // fp16, each value rounded to nearest even once; products without residual only.
   int h16;
 };
 
-// Eight fp32 values as three bf16 terms each, x = h + m + l exactly (8 + 8 + 8 significant
-// bits, each term the rest rounded to nearest).
+// Eight fp32 values as three bf16 terms each (8 + 8 + 8 significant bits, each term the rest
+// rounded to nearest): x = h + m + l exactly for |x| >= 2^-103 and within 2^-134 below (half the
+// spacing of bf16's subnormals, which the MFMA takes and gives as they are).  Where |x| rounds past
+// bf16's range, h is infinite and m and l are NaN.
 struct Split {
   bf16x8_t h, m, l;
 };
@@ -109,7 +118,9 @@ __device__ __forceinline__ Split split_bf16x3(float4 u, float4 v) {
           as_bf16x8(make_uint4(l[0], l[1], l[2], l[3]))};
 }
 
-template <int BM, int BN, int WK, bool VEC, bool GLU>
+// LONG: K from 2^24 on, where 64 rows no longer fit 32-bit byte offsets: the same loads by 64-bit
+// addresses.
+template <int BM, int BN, int WK, bool VEC, bool GLU, bool LONG>
 __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   constexpr int NT = 64 * WK;
   constexpr int FM = BM / 16, FN = BN / 16;
@@ -186,7 +197,16 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       }
       const __amdgpu_buffer_rsrc_t rs = is_a ? rs_a : t - BM < BW ? rs_w : rs_g;
       const auto dst = (__attribute__((address_space(3))) void*)(mine + t * kSK);
-      if constexpr (VEC)
+      if constexpr (LONG) {
+        const int c = (lane % LPR) / (VEC ? 1 : 4) ^ swz(lds_row);
+        const int k = s * kSK + (VEC ? 4 * c : 4 * c + lane % 4);
+        const float* src = (is_a ? a_row(row) : w_row(row + (t - BM) / BW * BW)) + min(k, K - 1);
+        const auto from = (__attribute__((address_space(1))) void*)(src);
+        if constexpr (VEC)
+          __builtin_amdgcn_global_load_lds(from, dst, 16, 0, 0);
+        else
+          __builtin_amdgcn_global_load_lds(from, dst, 4, 0, 0);
+      } else if constexpr (VEC)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 16, off, soff, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, off, soff, 0, 0);
@@ -201,13 +221,19 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int n_sl = a.chain ? 0 : (K + kSK - 1) / kSK;
+  const int n_sl = K / kSK + (K % kSK != 0);
+  // Sum of h * 2^96 over every operand of the wave, one MFMA per fragment: not finite once an
+  // operand reaches 2^32 (or the sum does): a product that overflows stays infinite or becomes NaN,
+  // also beside its opposite in one MFMA (measured for every pair of places).
+  f32x4_t guard = {0.f, 0.f, 0.f, 0.f};
+  constexpr uint32_t kGuard = 0x6f806f80u;
+  const bf16x8_t big = as_bf16x8(make_uint4(kGuard, kGuard, kGuard, kGuard));
   if (wave < n_sl) dma(wave);
   for (int s = wave; s < n_sl; s += WK) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // The whole slice to registers as bf16 terms, then the next slice's loads under the MFMAs:
     // the six products of terms that reach fp32's precision (the dropped m l, l m and l l are
-    // below 2^-26 of |x w|), smallest first.  The W fragment is the MFMA's row operand, so a
+    // below 2^-24 of |x w|), smallest first.  The W fragment is the MFMA's row operand, so a
     // lane ends up with 4 consecutive columns of one output row.
     float4 raw_a[FM][2], raw_w[FN][2];
     auto fetch = [&](float4(&raw)[2], int t) {
@@ -221,13 +247,31 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
 #pragma unroll
     for (int i = 0; i < FM; ++i) fetch(raw_a[i], 16 * i);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (s + WK < n_sl) dma(s + WK);
+    if (n_sl - s > WK) dma(s + WK);
+    if (LONG && !VEC && s == n_sl - 1) {  // elements past K came as copies of the last one
+      auto mask = [&](float4(&raw)[2]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int left = K - (s * kSK + 16 * h + 4 * fg);
+          raw[h] = make_float4(left > 0 ? raw[h].x : 0.f, left > 1 ? raw[h].y : 0.f,
+                               left > 2 ? raw[h].z : 0.f, left > 3 ? raw[h].w : 0.f);
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < FN; ++j) mask(raw_w[j]);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) mask(raw_a[i]);
+    }
     Split sa[FM];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) sa[i] = split_bf16x3(raw_a[i][0], raw_a[i][1]);
+    for (int i = 0; i < FM; ++i) {
+      sa[i] = split_bf16x3(raw_a[i][0], raw_a[i][1]);
+      guard = __builtin_amdgcn_mfma_f32_16x16x32_bf16(big, sa[i].h, guard, 0, 0, 0);
+    }
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const Split w = split_bf16x3(raw_w[j][0], raw_w[j][1]);
+      guard = __builtin_amdgcn_mfma_f32_16x16x32_bf16(big, w.h, guard, 0, 0, 0);
       auto mma = [&](const bf16x8_t& x, auto term) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -241,45 +285,141 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       mma(w.h, &Split::h);
     }
   }
-
   // Per-wave partial tiles to LDS, then the sum over the waves (in wave order) and the
   // epilogue, a thread per 4 columns
+  float low = INFINITY, odd = 0.0f;  // the smallest magnitude; NaN where a value is not finite
+  auto part = [&](int i, int j) -> f32x4_t& {
+    return *reinterpret_cast<f32x4_t*>(mine + (16 * i + fr) * kCLd + 16 * j + 4 * fg);
+  };
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-      *reinterpret_cast<f32x4_t*>(mine + (16 * i + fr) * kCLd + 16 * j + 4 * fg) = acc[i][j];
+    for (int j = 0; j < FN; ++j) {
+      part(i, j) = acc[i][j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        low = fminf(low, fabsf(acc[i][j][e]));
+        odd = fmaf(acc[i][j][e], 0.0f, odd);
+      }
+    }
+  float wide = 0.0f;  // NaN after an operand of 2^32 or more
+#pragma unroll
+  for (int e = 0; e < 4; ++e) wide = fmaf(guard[e], 0.0f, wide);
+  // Operands below 2^-103, whose terms do not sum to them, cost a value at most K 2^-101 while the
+  // others stay below 2^32: below 2^-26 of it from `small` on.  Smaller ones, ones that are not
+  // finite and, after an operand of 2^32 or more, all are formed again from the fp32 operands.
+  const float small = static_cast<float>(K) * 0x1p-75f;
+  if (wave < n_sl && __any(odd + wide != 0.0f || low < small)) [[unlikely]] {
+    // straight from memory; group fg takes floats 4 fg .. 4 fg + 3 of half a slice
+    auto load = [&](const float* row, int k) {
+      if (VEC) return *reinterpret_cast<const float4*>(row + k);
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = row[min(k + e, K - 1)];  // no branch: the loads are all in flight together
+        v[e] = k + e < K ? v[e] : 0.0f;
+      }
+      return make_float4(v[0], v[1], v[2], v[3]);
+    };
+    const bool all = __any(wide != 0.0f);
+    float least = INFINITY;  // of the values other than zero
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = fabsf(part(i, j)[e]);
+          least = v != 0.0f ? fminf(least, v) : least;
+        }
+    bool again = LONG || all || __any(odd != 0.0f || least < small);
+    if (!again) {  // zeros: right unless there are operands below 2^-103 other than zero
+      uint32_t key = 0xffffffffu;  // least 2 |bits| - 1: zeros last
+      constexpr int RPI = VEC ? 8 : 2, LPR = 64 / RPI, Q = (BM + BN) / RPI;
+#pragma unroll 1
+      for (int s = wave; s < n_sl; s += WK) {
+        // past the last row a buffer load gives zero; past K the last element serves
+        const uint32_t off =
+            lane / LPR * row_bytes +
+            (VEC ? s * (4 * kSK) + 16 * (lane % LPR) : 4 * min(s * kSK + lane % LPR, K - 1));
+        typename std::conditional_t<VEC, u32x4_t, uint32_t> x[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const int t = q * RPI;  // tile row of the instruction: A rows, then W rows
+          const __amdgpu_buffer_rsrc_t rs = t < BM ? rs_a : t - BM < BW ? rs_w : rs_g;
+          const uint32_t at = off + (t < BM ? t : (t - BM) % BW) * row_bytes;
+          if constexpr (VEC)
+            x[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0);
+          else
+            x[q] = __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          if constexpr (VEC) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) key = min(key, 2 * x[q][e] - 1);
+          } else {
+            key = min(key, 2 * x[q] - 1);
+          }
+        }
+      }
+      again = __any(key < 2 * __float_as_uint(0x1p-103f) - 1);
+    }
+    if (again) {
+      f32x4_t ex[FM][FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) ex[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // the next half on its way under the current one's MFMAs
+      float4 next_a[FM], next_w[FN];
+      auto fetch = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) next_a[i] = load(a_row(16 * i + fr), k + 4 * fg);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) next_w[j] = load(w_row(16 * j + fr), k + 4 * fg);
+      };
+      fetch(wave * kSK);
+#pragma unroll 1
+      for (int h = 0, s = wave; s < n_sl; s += WK * h, h ^= 1) {
+        float4 va[FM], vw[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) va[i] = next_a[i];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) vw[j] = next_w[j];
+        if (h == 0)
+          fetch(s * kSK + kSK / 2);
+        else if (n_sl - s > WK)
+          fetch((s + WK) * kSK);
+        auto mma = [&](auto f) {
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              ex[i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(vw[j].*f, va[i].*f, ex[i][j], 0, 0, 0);
+        };
+        mma(&float4::x), mma(&float4::y), mma(&float4::z), mma(&float4::w);
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          f32x4_t v = part(i, j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (all || !(fabsf(v[e]) >= small && fabsf(v[e]) < INFINITY)) v[e] = ex[i][j][e];
+          part(i, j) = v;
+        }
+    }
+  }
   __syncthreads();
-  // A value that is not finite (an infinite or NaN operand, one that rounds past bf16's range,
-  // an overflow), or so small that operands below 2^-109, whose third terms fall between bf16's
-  // subnormal numbers, may be behind it, is formed again as one fp32 chain.
-  auto suspect = [&](float t) {
-    const float mag = fabsf(t);
-    return !(mag < INFINITY) || (mag < 0x1p-90f && mag != 0.0f) || a.chain;
-  };
-  auto chain = [&](int r, int c) {
-    const float* x = a_row(r);
-    const float* y = w_row(c);
-    float t = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < K; ++k) t = fmaf(x[k], y[k], t);
-    return t;
-  };
   auto total = [&](int r, int c, float (&v)[4]) {
     f32x4_t t = *reinterpret_cast<const f32x4_t*>(smem[0] + r * kCLd + c);
 #pragma unroll
     for (int w = 1; w < WK; ++w) t += *reinterpret_cast<const f32x4_t*>(smem[w] + r * kCLd + c);
-    bool any = false;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      v[q] = t[q];
-      any |= suspect(t[q]);
-    }
-    if (any) [[unlikely]] {
-#pragma unroll 1
-      for (int q = 0; q < 4; ++q)
-        if (suspect(v[q])) v[q] = chain(r, c + q);
-    }
+    for (int q = 0; q < 4; ++q) v[q] = t[q];
   };
   if constexpr (GLU) {
     // columns [0, BN/2) of the tile are the value outputs of channels c0 .., [BN/2, BN) the
@@ -363,19 +503,12 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   constexpr int U = BM / RPS < 4 ? BM / RPS : 4;
   for (int r0 = tid / BN; r0 < BM && m0 + r0 < M; r0 += U * RPS) {
     float v[U];
-    bool any = false;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int r = r0 + u * RPS;
       v[u] = smem[0][r * kCLd + c];
 #pragma unroll
       for (int w = 1; w < WK; ++w) v[u] += smem[w][r * kCLd + c];
-      any |= suspect(v[u]);
-    }
-    if (any) [[unlikely]] {
-#pragma unroll 1
-      for (int u = 0; u < U; ++u)
-        if (suspect(v[u])) v[u] = chain(r0 + u * RPS, c);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -391,11 +524,11 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   }
 }
 
-template <int BM, int BN, int WK, bool VEC, bool GLU>
+template <int BM, int BN, int WK, bool VEC, bool GLU, bool LONG = false>
 int launch_tile(const SgemmArgs& a, hipStream_t s) {
   const int bn = GLU ? BN / 2 : BN, cols = GLU ? a.glu_c : a.N;
   const dim3 grid((cols + bn - 1) / bn, (a.M + BM - 1) / BM, a.batch);
-  hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WK, VEC, GLU>), grid, dim3(64 * WK), 0, s, a);
+  hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WK, VEC, GLU, LONG>), grid, dim3(64 * WK), 0, s, a);
   return check_launch("sgemm_nt_kernel");
 }
 
@@ -415,6 +548,7 @@ int launch_sized(const SgemmArgs& a, hipStream_t s) {
   auto tiles = [&](int bm, int bn) {
     return static_cast<long>((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
   };
+  if (a.K >= 1 << 24) return launch_tile<32, 32, 8, VEC, GLU, true>(a, s);
   if (a.K >= 1024) {
     if (tiles(32, 32) <= cus) return launch_tile<32, 32, 8, VEC, GLU>(a, s);
     if (tiles(32, 64) <= 2 * cus) return launch_tile<32, 64, 8, VEC, GLU>(a, s);
@@ -432,7 +566,6 @@ int launch_sized(const SgemmArgs& a, hipStream_t s) {
 
 int run_sgemm(SgemmArgs a, int batch, bool glu, hipStream_t s) {
   a.batch = batch;
-  a.chain = a.K >= (1 << 24);  // 64 rows of K floats past 4 GB
   const int rc = glu ? launch_sized<true, true>(a, s)
                  : a.vec ? launch_sized<true, false>(a, s) : launch_sized<false, false>(a, s);
   if (rc || !a.ln_g) return rc;

@@ -3,7 +3,7 @@ slices and dispatch, and on values outside bf16's range.
 
 Bound: an MFMA adds 32 products and the accumulator and rounds to fp32, at worst 2 ulp of the
 partial sum (<= 2^-22 sum|x w|); six MFMAs per 32-wide slice, then one addition per wave (8 at
-most) and the bias.  The split itself is exact but for terms below 2^-26 |x w|.  So
+most) and the bias.  The split itself is exact but for products of terms below 2^-24 |x w|.  So
 |got - truth| <= (6 ceil(K / 32) + 10) 2^-22 (sum|x w| + |bias|)."""
 from __future__ import annotations
 
@@ -24,6 +24,10 @@ def _run(x, w, bias):
     say("sgemm split", M, K, N)
     gemm.LaunchSgemm(up(x), up(w), None if bias is None else up(bias), out, M, K, N, 0)
     return down(out, (M, N))
+
+
+def _rel(got, ref):
+    return np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref)
 
 
 # one K below a slice; K a slice and a part; the limits of the K classes (255 / 256, 1023 / 1024);
@@ -76,9 +80,51 @@ def test_sgemm_split_special_values():
         assert np.all(err <= K * (2.0 ** -23 * mag[ok] + 2.0 ** -149))
 
 
+# x and w scaled by powers of two whose products are ordinary numbers: below 2^-103 an operand's
+# third bf16 term falls between bf16's subnormals, below 2^-134 all three are zero
+@pytest.mark.parametrize("ex,ew", [(-102, 40), (-110, 60), (-118, 40), (-125, 60), (-135, 60),
+                                   (-140, 100), (-147, 120), (60, -135), (100, -140), (-118, 0)])
+@pytest.mark.parametrize("M,K,N", [(33, 512, 70), (40, 290, 65), (3, 64, 5), (70, 1024, 2050)])
+def test_sgemm_operands_outside_the_terms_range(M, K, N, ex, ew):
+    """As close to fp64 as the fp32 MFMAs that form these results (2.9e-7 on ordinary operands);
+    operands are exact inputs, so only the products and sums round.  Half of x's rows and a third
+    of its columns are zero: a zero result must not pass for an exact one."""
+    r = SplitMix64(M + K + N)
+    x = np.ldexp(r.normal((M, K)), ex).astype(np.float32)
+    w = np.ldexp(r.normal((N, K)), ew).astype(np.float32)
+    x[1::2] = 0
+    x[:, ::3] = 0
+    got = _run(x, w, None)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.all(got[1::2] == 0)
+    assert _rel(got, ref) <= 4e-7
+
+
+def test_sgemm_tiny_operand_beside_ordinary_ones():
+    """One tiny and one huge operand in a row of ordinary ones, their product the largest term."""
+    r = SplitMix64(8)
+    M, K, N = 35, 320, 37
+    x, w = r.normal((M, K)), r.normal((N, K))
+    x[:, 77] = np.float32(1.2345678 * 2.0 ** -120)
+    w[:, 77] = np.float32(1.7 * 2.0 ** 126)
+    got = _run(x, w, None)
+    assert _rel(got, x.astype(np.float64) @ w.astype(np.float64).T) <= 4e-7
+
+
+def test_sgemm_finite_near_the_largest_number():
+    """Operands whose first terms' product overflows although the product does not."""
+    x = np.full((2, 1), np.float32(2.0 ** 64 * (1 - 2.0 ** -20)))
+    got = _run(x, x, None)
+    np.testing.assert_array_equal(got, x * x.T)
+    assert np.all(np.isfinite(got))
+
+
 def test_sgemm_split_rows_past_32_bit_offsets():
-    """K >= 2^24: 64 rows no longer fit 32-bit byte offsets; integer operands, exact sum."""
+    """K >= 2^24: 64 rows no longer fit 32-bit byte offsets; integer operands, exact sum.  And all
+    threes: a single chain rounds each addition above 2^24, parts of K stay exact."""
     K = (1 << 24) + 5
+    got = _run(np.full((1, K), 3, np.float32), np.ones((1, K), np.float32), None)
+    assert abs(float(got[0, 0]) - 3 * K) <= 2.0 ** -22 * 3 * K
     r = np.random.default_rng(3)
     x = r.integers(-1, 2, (1, K)).astype(np.float32)
     w = r.integers(-1, 2, (2, K)).astype(np.float32)
