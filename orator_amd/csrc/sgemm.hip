@@ -7,10 +7,10 @@
 // fp32 products on the bf16 matrix cores: every operand is split in registers into three bf16
 // terms, whose sum is the fp32 value exactly from 2^-103 on, and the six products of terms that
 // reach fp32's precision are accumulated in fp32 (what is dropped is below 2^-24 of |x w|, and the
-// MFMA adds 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96 cycles
-// per 16 x 16 x 32 block, the fp32 MFMA's 256.  Measured against 64 bits (random normal
-// operands, relative 2-norm): K = 512 0.8-1.2e-7, K = 2048 1.7e-7, K = 64 4.7e-8; the fp32 MFMA
-// 2.9e-7 unsplit (2.1e-7 with K in two parts), 2.1e-7 in eight parts, 1.4e-7.
+// MFMA adds 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96
+// cycles per 16 x 16 x 32 block, the fp32 MFMA's 256.  Measured against 64 bits (random normal
+// operands, relative 2-norm; the fp32 MFMA in parentheses): K = 64 4.7e-8 (1.4e-7), 255 1.6e-7
+// (2.9e-7), 512 1.6e-7 (4.1e-7), 2048 2.4e-7 (2.9e-7 in eight parts).
 //
 // Results that the terms cannot carry are formed again by the wave on the fp32 MFMA: those that are
 // not finite, those so small that operands below 2^-103 may show in them, and all after an operand
@@ -34,11 +34,15 @@
 // scheduling groups and wave priorities: no effect.
 //
 // Measured (us, replayed launches; before: the fp32-MFMA kernel with split K and its reduction):
-//   717 x 512 -> 2048  28.7 -> 16.3   717 x 2048 -> 512  24.5 -> 17.3   717 x 512 -> 512 12.2 -> 8.2
-//   717 x 512 -> 1536  27.0 -> 15.1   1433 x 512 -> 512  15.4 -> 10.6   717 x 512 -> 1024 15.4 -> 10.8
-//   126 x 512 -> 2048  11.2 -> 5.9    126 x 2048 -> 512  12.7 -> 11.9   126 x 512 -> 512 10.3 -> 5.8
-//   8 x (717 x 717 -> 64) 19.8 -> 14.1; 8 x (717 x 64 -> 717) 14.2 -> 14.1, 8 x (1000 x 64 -> 1999)
-//   31.2 -> 36.6 (bound by its 64 MB of unaligned rows written).
+//   717 x 512 -> 2048   24.9 -> 15.5    717 x 2048 -> 512   25.1 -> 18.2
+//   717 x 512 -> 512    12.4 -> 8.0     717 x 512 -> 1536   24.5 -> 14.6
+//   1433 x 512 -> 512   15.6 -> 10.6    717 x 512 -> 1024   15.3 -> 10.3
+//   126 x 512 -> 2048   11.6 -> 6.1     126 x 2048 -> 512   12.7 -> 11.9
+//   126 x 512 -> 512    10.5 -> 5.7     8 x (717 x 717 -> 64)  20.3 -> 13.6
+//   8 x (717 x 64 -> 717)  14.2 -> 13.2
+//   8 x (1000 x 64 -> 1999)  33.1 -> 28.9 (64 MB of unaligned rows written)
+// Behind it still: a few rows at K < 32, which take element loads (8 x (16 x 16 -> 64) 4.2 -> 4.8),
+// and 8 x (503 x 64 -> 1005), 11.2 -> 11.7.
 #include <stdint.h>
 
 #include <algorithm>
@@ -69,7 +73,9 @@ struct SgemmArgs {
   const float* bias;
   float* out;
   int M, K, N, act;
-  int batch;  // blockIdx.z = batch entry
+  int batch;
+  int tiles_n, tiles_m;        // of one batch entry
+  uint32_t rec_tiles, rec_run;  // floor(2^32 / d) of their product and of the faster running one
   long s_in, s_w, s_out;
   bool vec;  // K % 32 == 0 and 16-byte aligned operands: 16-byte loads
   // Grouped products (group > 0): `group` problems share `in`; problem z uses weight Wg[z],
@@ -135,14 +141,22 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   // Workgroups are dealt to the 8 XCDs in turn: give each a contiguous piece of the tile order
   // (batch entries, then tiles with the operand of more rows running slowest), so the tiles that
   // share an L2 share rows of it, and the lines that neighbours write in part meet there.
-  const int gx = gridDim.x, gy = gridDim.y, total_wg = gx * gy * static_cast<int>(gridDim.z);
-  const int lin = blockIdx.x + gx * (blockIdx.y + gy * static_cast<int>(blockIdx.z));
-  const int xcd = lin & 7;
-  const int at = xcd * (total_wg >> 3) + min(xcd, total_wg & 7) + (lin >> 3);
-  const int batch = at / (gx * gy), in_batch = at - batch * (gx * gy);
+  const uint32_t total = gridDim.x * gridDim.y * gridDim.z;
+  const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const uint32_t xcd = lin & 7;
+  const uint32_t at = xcd * (total >> 3) + min(xcd, total & 7) + (lin >> 3);
   const bool n_slow = a.N > a.M;
-  const int tile_n = n_slow ? in_batch / gy : in_batch % gx;
-  const int tile_m = n_slow ? in_batch % gy : in_batch / gx;
+  // n / d by its reciprocal, at most one short (scalar instructions; the compiler's own division
+  // is a chain of vector ones)
+  auto div = [](uint32_t n, uint32_t d, uint32_t rec) {
+    const uint32_t q = __umulhi(n, rec);
+    return q + (n - q * d >= d);
+  };
+  const uint32_t per_batch = a.tiles_n * a.tiles_m, run = n_slow ? a.tiles_m : a.tiles_n;
+  const int batch = a.batch == 1 ? 0 : div(at, per_batch, a.rec_tiles);
+  const uint32_t in_batch = at - batch * per_batch;
+  const int slow = div(in_batch, run, a.rec_run), fast = in_batch - slow * run;
+  const int tile_n = n_slow ? slow : fast, tile_m = n_slow ? fast : slow;
   const float* A = a.in + batch * a.s_in;
   const float* B = a.group ? a.Wg[batch] : a.W + batch * a.s_w;
   const int M = a.M, N = a.N, K = a.K;
@@ -183,8 +197,7 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
     for (int q = 0; q < (BM + BN) / RPI; ++q) {
       const int t = q * RPI;  // tile row of the instruction: A rows, then W rows
       const bool is_a = t < BM;
-      const int first = is_a ? t : (t - BM) % BW;
-      const int r = first + lane / LPR;
+      const int r = (is_a ? t : (t - BM) % BW) + lane / LPR;
       const int row = min(r, (is_a ? rows_a : rows_w) - 1);
       const int lds_row = t + lane / LPR;
       uint32_t off, soff = 0;
@@ -200,7 +213,8 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       if constexpr (LONG) {
         const int c = (lane % LPR) / (VEC ? 1 : 4) ^ swz(lds_row);
         const int k = s * kSK + (VEC ? 4 * c : 4 * c + lane % 4);
-        const float* src = (is_a ? a_row(row) : w_row(row + (t - BM) / BW * BW)) + min(k, K - 1);
+        const float* src =
+            (is_a ? a_row(row) : w_row(row + (t - BM) / BW * BW)) + min(k, K - 1);
         const auto from = (__attribute__((address_space(1))) void*)(src);
         if constexpr (VEC)
           __builtin_amdgcn_global_load_lds(from, dst, 16, 0, 0);
@@ -216,10 +230,11 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   // 16 + 4g .. of the slice (the same k for A and W, so any assignment serves)
   const int fr = lane & 15, fg = lane >> 4;
   f32x4_t acc[FM][FN];
+  [[maybe_unused]] f32x4_t sum[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FN; ++j) sum[i][j] = acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int n_sl = K / kSK + (K % kSK != 0);
   // Sum of h * 2^96 over every operand of the wave, one MFMA per fragment: not finite once an
@@ -248,7 +263,7 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
     for (int i = 0; i < FM; ++i) fetch(raw_a[i], 16 * i);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (n_sl - s > WK) dma(s + WK);
-    if (LONG && !VEC && s == n_sl - 1) {  // elements past K came as copies of the last one
+    if (LONG && !VEC && s >= K / kSK) {  // elements past K came as copies of the last one
       auto mask = [&](float4(&raw)[2]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -284,6 +299,21 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       mma(w.h, &Split::m);
       mma(w.h, &Split::h);
     }
+    if constexpr (WK == 1) {  // (two slices at most) as two waves would add them
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
   }
   // Per-wave partial tiles to LDS, then the sum over the waves (in wave order) and the
   // epilogue, a thread per 4 columns
@@ -414,7 +444,7 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
     }
   }
   __syncthreads();
-  auto total = [&](int r, int c, float (&v)[4]) {
+  auto total_of = [&](int r, int c, float (&v)[4]) {
     f32x4_t t = *reinterpret_cast<const f32x4_t*>(smem[0] + r * kCLd + c);
 #pragma unroll
     for (int w = 1; w < WK; ++w) t += *reinterpret_cast<const f32x4_t*>(smem[w] + r * kCLd + c);
@@ -441,8 +471,8 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       const int m = m0 + r;
       if (m >= M) continue;
       float av[4], gv[4], o[4];
-      total(r, j, av);
-      total(r, HB + j, gv);
+      total_of(r, j, av);
+      total_of(r, HB + j, gv);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float x = av[q] + ba[q], g = gv[q] + bg[q];
@@ -462,10 +492,15 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   float* C = a.group ? a.og[batch] : a.out + batch * a.s_out;
   const float* bias = a.group ? a.bg[batch] : a.bias;
   const bool h16 = (a.h16 >> (a.group ? batch : 0)) & 1;
-  auto finish = [&](float v, float b, const float* old) {
+  // The rows in two forms: without options, and with every option looked at per element (8 x (717 x
+  // 64 -> 1433): 22.8 us, 19.4 without, scalar division included).
+  const bool plain = !a.act && !a.residual && !h16;
+  auto finish = [&](float v, float b, const float* old, auto simple) {
+    if constexpr (simple) return v + b;
     v = apply_act(v + b, a.act);
     return a.residual ? fmaf(a.res_scale, v, *old) : v;
   };
+  const int rows = min(BM, M - m0);
   if ((N % 4) == 0 && (reinterpret_cast<uintptr_t>(C) & (h16 ? 7 : 15)) == 0) {
     // 4 columns per thread, one 16-byte (fp16: 8-byte) store
     constexpr int TPRo = BN / 4, RPIo = NT / TPRo;
@@ -477,21 +512,24 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) bv[q] = bias[n + q];
     }
-    for (int r = orow; r < BM && m0 + r < M; r += RPIo) {
-      const long at = static_cast<long>(m0 + r) * N + n;
-      float v[4];
-      total(r, ocol, v);
+    auto store = [&](auto simple) {
+      for (int r = orow; r < rows; r += RPIo) {
+        const long at = static_cast<long>(m0 + r) * N + n;
+        float v[4];
+        total_of(r, ocol, v);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = finish(v[q], bv[q], C + at + q);
-      if (h16) {
-        typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
-        const h4_t hv = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]),
-                         static_cast<_Float16>(v[2]), static_cast<_Float16>(v[3])};
-        *reinterpret_cast<h4_t*>(reinterpret_cast<_Float16*>(C) + at) = hv;
-      } else {
-        *reinterpret_cast<float4*>(C + at) = make_float4(v[0], v[1], v[2], v[3]);
+        for (int q = 0; q < 4; ++q) v[q] = finish(v[q], bv[q], C + at + q, simple);
+        if (!simple && h16) {
+          typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+          const h4_t hv = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]),
+                           static_cast<_Float16>(v[2]), static_cast<_Float16>(v[3])};
+          *reinterpret_cast<h4_t*>(reinterpret_cast<_Float16*>(C) + at) = hv;
+        } else {
+          *reinterpret_cast<float4*>(C + at) = make_float4(v[0], v[1], v[2], v[3]);
+        }
       }
-    }
+    };
+    plain ? store(std::true_type{}) : store(std::false_type{});
     return;
   }
   // other row lengths and alignments: a column per thread, so that a store instruction still
@@ -501,47 +539,59 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   if (n >= N) return;
   const float b = bias ? bias[n] : 0.0f;
   constexpr int U = BM / RPS < 4 ? BM / RPS : 4;
-  for (int r0 = tid / BN; r0 < BM && m0 + r0 < M; r0 += U * RPS) {
-    float v[U];
+  auto store = [&](auto simple) {
+    for (int r0 = tid / BN; r0 < rows; r0 += U * RPS) {
+      float v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int r = r0 + u * RPS;
-      v[u] = smem[0][r * kCLd + c];
+      for (int u = 0; u < U; ++u) {
+        const int r = r0 + u * RPS;
+        v[u] = smem[0][r * kCLd + c];
 #pragma unroll
-      for (int w = 1; w < WK; ++w) v[u] += smem[w][r * kCLd + c];
+        for (int w = 1; w < WK; ++w) v[u] += smem[w][r * kCLd + c];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = r0 + u * RPS;
+        if (r >= rows) break;
+        const long at = static_cast<long>(m0 + r) * N + n;
+        const float x = finish(v[u], b, C + at, simple);
+        if (!simple && h16)
+          reinterpret_cast<_Float16*>(C)[at] = static_cast<_Float16>(x);
+        else
+          C[at] = x;
+      }
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int m = m0 + r0 + u * RPS;
-      if (m >= M) break;
-      const long at = static_cast<long>(m) * N + n;
-      const float x = finish(v[u], b, C + at);
-      if (h16)
-        reinterpret_cast<_Float16*>(C)[at] = static_cast<_Float16>(x);
-      else
-        C[at] = x;
-    }
-  }
+  };
+  plain ? store(std::true_type{}) : store(std::false_type{});
 }
 
 template <int BM, int BN, int WK, bool VEC, bool GLU, bool LONG = false>
-int launch_tile(const SgemmArgs& a, hipStream_t s) {
+int launch_tile(SgemmArgs a, hipStream_t s) {
   const int bn = GLU ? BN / 2 : BN, cols = GLU ? a.glu_c : a.N;
-  const dim3 grid((cols + bn - 1) / bn, (a.M + BM - 1) / BM, a.batch);
+  a.tiles_n = (cols + bn - 1) / bn;
+  a.tiles_m = (a.M + BM - 1) / BM;
+  auto rec = [](uint64_t d) {
+    return static_cast<uint32_t>(std::min<uint64_t>((1ull << 32) / d, 0xffffffffu));
+  };
+  a.rec_tiles = rec(static_cast<uint64_t>(a.tiles_n) * a.tiles_m);
+  a.rec_run = rec(a.N > a.M ? a.tiles_m : a.tiles_n);
+  const dim3 grid(a.tiles_n, a.tiles_m, a.batch);
   hipLaunchKernelGGL((sgemm_nt_kernel<BM, BN, WK, VEC, GLU, LONG>), grid, dim3(64 * WK), 0, s, a);
   return check_launch("sgemm_nt_kernel");
 }
 
 // Tile and waves by K and grid.  Many small tiles keep every CU busy where the grid is short;
 // larger tiles split fewer elements per MFMA.  Eight waves per tile shorten a short grid's time
-// (126 x 512 -> 512: 5.8 us, 6.1 with four) and, for long K, keep the partial sums short (K =
-// 2048: error 1.7e-7, four waves 2.4e-7); four let two to five workgroups share a CU, so that
-// one's first loads and epilogue run under the others' MFMAs (717 x 512 -> 2048: 32 x 64 tiles,
-// four waves 17.5 us, eight 20.8; 2000 x 512 -> 2048: 64 x 64, four waves 34.6, eight 43.3, 32 x
-// 64 38.3; 717 x 512 -> 1536: 32 x 32, four waves 15.8, eight 17.3, 32 x 64 16.2; 717 x 2048 ->
-// 512: 32 x 64, eight waves 17.6, 32 x 32 20.0, 64 x 64 25.6).  Short K (few slices per tile): 32 x 32
-// tiles, bound by the outputs written (8 x (717 x 64 -> 717): two waves 14.1 us, 32 x 64 15.8,
-// 64 x 64 21.7).
+// (126 x 512 -> 512: 5.8 us, 6.1 with four) and, for long K, keep the partial sums short; four let
+// two to five workgroups share a CU, so that one's first loads and epilogue run under the others'
+// MFMAs (717 x 512 -> 2048: 32 x 64 tiles, four waves 17.5 us, eight 20.8; 2000 x 512 -> 2048: 64 x
+// 64, four waves 34.6, eight 43.3, 32 x 64 38.3; 717 x 512 -> 1536: 32 x 32, four waves 15.8, eight
+// 17.3, 32 x 64 16.2; 717 x 2048 -> 512: 32 x 64, eight waves 17.6, 32 x 32 20.0, 64 x 64 25.6).
+// Short K: the instructions around the few slices and the outputs bound it, so 32 x 32 tiles with a
+// wave per slice while the grid is short, then wave tiles of 32 x 64, from 15 tiles per CU on one
+// wave for both slices (8 x (600 x 64 -> 600): 32 x 32 with two waves 9.5 us, 32 x 64 with two 8.4;
+// 8 x (1000 x 64 -> 1999): 32 x 32 two waves 31.6, 32 x 64 two 32.4, one 28.5; 1999 x 30 -> 2048:
+// 13.9 and, one wave, 10.7).
 template <bool VEC, bool GLU>
 int launch_sized(const SgemmArgs& a, hipStream_t s) {
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
@@ -560,7 +610,14 @@ int launch_sized(const SgemmArgs& a, hipStream_t s) {
     if (tiles(32, 64) <= 4 * cus) return launch_tile<32, 64, 4, VEC, GLU>(a, s);
     return launch_tile<64, 64, 4, VEC, GLU>(a, s);
   }
-  if (tiles(32, 32) <= 4 * cus) return launch_tile<32, 32, 4, VEC, GLU>(a, s);
+  const long t = tiles(32, 32);
+  if (a.K <= kSK) {
+    if (t <= 8 * cus) return launch_tile<32, 32, 1, VEC, GLU>(a, s);
+    return launch_tile<32, 64, 1, VEC, GLU>(a, s);
+  }
+  if (t <= 4 * cus) return launch_tile<32, 32, 4, VEC, GLU>(a, s);
+  if (a.K <= 2 * kSK && t > 15 * cus) return launch_tile<32, 64, 1, VEC, GLU>(a, s);
+  if (a.K <= 2 * kSK && t > 8 * cus) return launch_tile<32, 64, 2, VEC, GLU>(a, s);
   return launch_tile<32, 32, 2, VEC, GLU>(a, s);
 }
 

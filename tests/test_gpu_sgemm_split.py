@@ -32,11 +32,13 @@ def _rel(got, ref):
 
 # one K below a slice; K a slice and a part; the limits of the K classes (255 / 256, 1023 / 1024);
 # ragged rows and columns of every tile (32 x 32 with 2, 4 and 8 waves, 32 x 64 and 64 x 64 with 4
-# and 8); 16-byte and element loads
+# and 8); 16-byte and element loads; the one-wave and two-wave 32 x 64 tiles of K <= 64
 @pytest.mark.parametrize("M,K,N", [(1, 1, 1), (33, 31, 31), (31, 33, 65), (97, 255, 130),
                                    (290, 64, 1100), (33, 256, 33), (300, 256, 1030),
                                    (700, 512, 2050), (2050, 290, 2047), (130, 1023, 70),
-                                   (129, 1024, 257), (520, 1056, 514), (1030, 1024, 1028)])
+                                   (129, 1024, 257), (520, 1056, 514), (1030, 1024, 1028),
+                                   (2049, 31, 1030), (1030, 32, 2050), (2100, 64, 1030),
+                                   (2049, 40, 2050), (4100, 64, 1028)])
 def test_sgemm_split_edges(M, K, N):
     r = SplitMix64(M + 3 * K + 7 * N)
     x, w, b = r.normal((M, K)), r.normal((N, K)), r.normal((N,))
