@@ -33,6 +33,10 @@ constexpr int kWsPrefill = 4;        // partials of the long-prompt prefill's cu
 constexpr int kWsPrefillArrive = 5;  // its arrival counters
 // *fresh (optional): the block was allocated by this call, its contents undefined.
 void* workspace(hipStream_t stream, size_t bytes, int slot = 0, bool* fresh = nullptr);
+
+// Whether workspace() serves `bytes` without allocating while `stream` is being captured (where HIP
+// refuses it): always when it is not.
+bool workspace_at_hand(hipStream_t stream, size_t bytes, int slot = 0);
 // Frees every workspace block of `stream` (all threads, current and retired) after the
 // stream's queued work; for the owner of a stream about to be destroyed.
 int workspace_release(hipStream_t stream);

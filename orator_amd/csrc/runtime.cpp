@@ -118,6 +118,13 @@ void* workspace(hipStream_t stream, size_t bytes, int slot, bool* fresh) {
   return p;
 }
 
+bool workspace_at_hand(hipStream_t stream, size_t bytes, int slot) {
+  int dev = 0;
+  if (check_hip(hipGetDevice(&dev), "hipGetDevice") != ORATOR_OK) return false;
+  return !ws_capturing(stream) ||
+         ws_pool().holds(WsKey{dev, stream, std::this_thread::get_id(), slot}, bytes);
+}
+
 int workspace_release(hipStream_t stream) {
   int dev = 0;
   if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;

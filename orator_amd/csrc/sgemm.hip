@@ -10,7 +10,8 @@
 // MFMA adds 32 products per rounding where an fp32 chain rounds at each).  Six bf16 MFMAs take 96
 // cycles per 16 x 16 x 32 block, the fp32 MFMA's 256.  Measured against 64 bits (random normal
 // operands, relative 2-norm; the fp32 MFMA in parentheses): K = 64 4.7e-8 (1.4e-7), 255 1.6e-7
-// (2.9e-7), 512 1.6e-7 (4.1e-7), 2048 2.4e-7 (2.9e-7 in eight parts).
+// (2.9e-7), 512 1.6e-7 (4.1e-7), 2048 2.4e-7 whole and 1.7e-7 split over workgroups (2.9e-7 in
+// eight parts), 4096 split 1.7e-7 (4.4e-7).
 //
 // Results that the terms cannot carry are formed again by the wave on the fp32 MFMA: those that are
 // not finite, those so small that operands below 2^-103 may show in them, and all after an operand
@@ -37,7 +38,7 @@
 //   717 x 512 -> 2048   24.9 -> 15.5    717 x 2048 -> 512   25.1 -> 18.2
 //   717 x 512 -> 512    12.4 -> 8.0     717 x 512 -> 1536   24.5 -> 14.6
 //   1433 x 512 -> 512   15.6 -> 10.6    717 x 512 -> 1024   15.3 -> 10.3
-//   126 x 512 -> 2048   11.6 -> 6.1     126 x 2048 -> 512   12.7 -> 11.9
+//   126 x 512 -> 2048   11.6 -> 6.1     126 x 2048 -> 512   12.7 -> 10.1
 //   126 x 512 -> 512    10.5 -> 5.7     8 x (717 x 717 -> 64)  20.3 -> 13.6
 //   8 x (717 x 64 -> 717)  14.2 -> 13.2
 //   8 x (1000 x 64 -> 1999)  33.1 -> 28.9 (64 MB of unaligned rows written)
@@ -74,6 +75,7 @@ struct SgemmArgs {
   float* out;
   int M, K, N, act;
   int batch;
+  int slices;  // K split over workgroups: batch entry z takes slices z * slices on; 0: not split
   int tiles_n, tiles_m;        // of one batch entry
   uint32_t rec_tiles, rec_run;  // floor(2^32 / d) of their product and of the faster running one
   long s_in, s_w, s_out;
@@ -236,15 +238,17 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) sum[i][j] = acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int n_sl = K / kSK + (K % kSK != 0);
+  const int n_all = K / kSK + (K % kSK != 0);
+  const int first = a.slices ? batch * a.slices + wave : wave;  // this wave's: first, + WK, ...
+  const int n_sl = a.slices ? min(n_all, (batch + 1) * a.slices) : n_all;
   // Sum of h * 2^96 over every operand of the wave, one MFMA per fragment: not finite once an
   // operand reaches 2^32 (or the sum does): a product that overflows stays infinite or becomes NaN,
   // also beside its opposite in one MFMA (measured for every pair of places).
   f32x4_t guard = {0.f, 0.f, 0.f, 0.f};
   constexpr uint32_t kGuard = 0x6f806f80u;
   const bf16x8_t big = as_bf16x8(make_uint4(kGuard, kGuard, kGuard, kGuard));
-  if (wave < n_sl) dma(wave);
-  for (int s = wave; s < n_sl; s += WK) {
+  if (first < n_sl) dma(first);
+  for (int s = first; s < n_sl; s += WK) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // The whole slice to registers as bf16 terms, then the next slice's loads under the MFMAs:
     // the six products of terms that reach fp32's precision (the dropped m l, l m and l l are
@@ -339,7 +343,7 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
   // others stay below 2^32: below 2^-26 of it from `small` on.  Smaller ones, ones that are not
   // finite and, after an operand of 2^32 or more, all are formed again from the fp32 operands.
   const float small = static_cast<float>(K) * 0x1p-75f;
-  if (wave < n_sl && __any(odd + wide != 0.0f || low < small)) [[unlikely]] {
+  if (first < n_sl && __any(odd + wide != 0.0f || low < small)) [[unlikely]] {
     // straight from memory; group fg takes floats 4 fg .. 4 fg + 3 of half a slice
     auto load = [&](const float* row, int k) {
       if (VEC) return *reinterpret_cast<const float4*>(row + k);
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
       uint32_t key = 0xffffffffu;  // least 2 |bits| - 1: zeros last
       constexpr int RPI = VEC ? 8 : 2, LPR = 64 / RPI, Q = (BM + BN) / RPI;
 #pragma unroll 1
-      for (int s = wave; s < n_sl; s += WK) {
+      for (int s = first; s < n_sl; s += WK) {
         // past the last row a buffer load gives zero; past K the last element serves
         const uint32_t off =
             lane / LPR * row_bytes +
@@ -409,9 +413,9 @@ __global__ __launch_bounds__(64 * WK, 2) void sgemm_nt_kernel(SgemmArgs a) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) next_w[j] = load(w_row(16 * j + fr), k + 4 * fg);
       };
-      fetch(wave * kSK);
+      fetch(first * kSK);
 #pragma unroll 1
-      for (int h = 0, s = wave; s < n_sl; s += WK * h, h ^= 1) {
+      for (int h = 0, s = first; s < n_sl; s += WK * h, h ^= 1) {
         float4 va[FM], vw[FN];
 #pragma unroll
         for (int i = 0; i < FM; ++i) va[i] = next_a[i];
@@ -621,9 +625,57 @@ int launch_sized(const SgemmArgs& a, hipStream_t s) {
   return launch_tile<32, 32, 2, VEC, GLU>(a, s);
 }
 
+// out[i] = act(sum_z part[z][i] + bias), z ascending, or the residual update.
+__global__ __launch_bounds__(256) void sgemm_reduce_kernel(SgemmArgs a, const float* part,
+                                                           int splits) {
+  const long MN = static_cast<long>(a.M) * a.N;
+  const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= MN) return;
+  float v = part[i];
+  for (int z = 1; z < splits; ++z) v += part[z * MN + i];
+  v = apply_act(v + (a.bias ? a.bias[i % a.N] : 0.0f), a.act);
+  a.out[i] = a.residual ? fmaf(a.res_scale, v, a.out[i]) : v;
+}
+
+// Long K on a short grid: parts of K, 1024 each at least, on workgroups of their own, as many as
+// the CUs take in one round, and a second launch that adds them (us, whole and split: 126 x 2048
+// -> 512 12.0 and 10.1, 1 x 4096 -> 1024 19.0 and 10.7, 64 x 16384 -> 64 65.7 and 13.4; one row and
+// two columns at K = 2^24 63 ms and 0.32).
+int run_split(const SgemmArgs& a, int splits, float* part, hipStream_t s) {
+  const int n_sl = a.K / kSK + (a.K % kSK != 0);
+  SgemmArgs p = a;
+  p.slices = (n_sl + splits - 1) / splits;
+  splits = (n_sl + p.slices - 1) / p.slices;
+  const long MN = static_cast<long>(a.M) * a.N;
+  p.out = part;
+  p.batch = splits;
+  p.s_out = MN;
+  p.bias = nullptr;
+  p.act = p.residual = 0;
+  const bool far = a.K >= 1 << 24;
+  const int rc = a.vec ? (far ? launch_tile<32, 32, 8, true, false, true>(p, s)
+                              : launch_tile<32, 32, 8, true, false>(p, s))
+                       : (far ? launch_tile<32, 32, 8, false, false, true>(p, s)
+                              : launch_tile<32, 32, 8, false, false>(p, s));
+  if (rc) return rc;
+  hipLaunchKernelGGL(sgemm_reduce_kernel, dim3(static_cast<unsigned>((MN + 255) / 256)), dim3(256),
+                     0, s, a, part, splits);
+  return check_launch("sgemm_reduce_kernel");
+}
+
 int run_sgemm(SgemmArgs a, int batch, bool glu, hipStream_t s) {
   a.batch = batch;
-  const int rc = glu ? launch_sized<true, true>(a, s)
+  const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const long tiles = static_cast<long>((a.M + 31) / 32) * ((a.N + 31) / 32);
+  const long splits = std::min<long>(cus / tiles, a.K / 1024);
+  float* part = nullptr;  // without room for it, as in a capture before the first call: not split
+  if (splits > 1 && batch == 1 && !glu && !a.h16) {
+    const size_t bytes = splits * sizeof(float) * a.M * a.N;
+    if (workspace_at_hand(s, bytes, kWsGemm))
+      part = static_cast<float*>(workspace(s, bytes, kWsGemm));
+  }
+  const int rc = part ? run_split(a, static_cast<int>(splits), part, s)
+                 : glu ? launch_sized<true, true>(a, s)
                  : a.vec ? launch_sized<true, false>(a, s) : launch_sized<false, false>(a, s);
   if (rc || !a.ln_g) return rc;
   return launch_layer_norm(a.out, a.ln_g, a.ln_b, a.ln_out, a.M, a.N, a.ln_eps, s);

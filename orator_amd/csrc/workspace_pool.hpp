@@ -91,6 +91,13 @@ class WorkspacePool {
     return p;
   }
 
+  // Whether get() would serve `bytes` from the block that k has now.
+  bool holds(const WsKey& k, size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu_);
+    const auto it = map_.find(k);
+    return it != map_.end() && it->second.ptr && it->second.bytes >= bytes;
+  }
+
   // Frees every block (current, retired, pending, all threads) of `stream` on device `dev`
   // after the stream's queued work has finished.  Returns the sync status (blocks are freed
   // either way: the caller is about to destroy the stream).

@@ -80,6 +80,7 @@ int main() {
   const WsKey a{0, s1, std::this_thread::get_id()};
   void* p1 = pool.get(a, 100, false, nullptr);
   CHECK(p1 && pool.get(a, 50, false, nullptr) == p1);  // fits: same block
+  CHECK(pool.holds(a, WorkspacePool::kGrain) && !pool.holds(a, WorkspacePool::kGrain + 1));
   g_queued[s1] = 1;                                    // work queued on p1
   void* p2 = pool.get(a, 1000000, false, nullptr);     // grows: new block, old one retired
   CHECK(p2 && p2 != p1 && g_live.count(p1) == 1 && pool.held_blocks() == 2);

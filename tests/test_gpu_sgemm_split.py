@@ -7,12 +7,15 @@ most) and the bias.  The split itself is exact but for products of terms below 2
 |got - truth| <= (6 ceil(K / 32) + 10) 2^-22 (sum|x w| + |bias|)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from gpu_helpers import down, empty, say, up
 from helpers import SplitMix64
 from orator_amd import gemm
+from orator_amd.runtime import Stream, synchronize
 
 pytestmark = pytest.mark.gpu
 
@@ -45,7 +48,71 @@ def test_sgemm_split_edges(M, K, N):
     got = _run(x, w, b)
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     bound = (6 * -(-K // 32) + 10) * 2.0 ** -22 * (np.abs(x64) @ np.abs(w64).T + np.abs(b))
-    assert np.all(np.abs(got - (x64 @ w64.T + b)) <= bound)
+    ref = x64 @ w64.T + b
+    assert np.all(np.abs(got - ref) <= bound)
+    # the sharper check: without the third terms or the corrections the error is 4e-6 and more
+    # (measured with all six products: 2.4e-7 at most)
+    assert _rel(got, ref) <= 4e-7
+
+
+# K split over workgroups: two parts, as many as one round takes, an uneven last one, element loads,
+# a tile of one row.  33 outputs at least: the 2-norm of the errors over that of the sums is then
+# near their ratio of standard deviations, where a single sum may cancel (one of 70000 products
+# that came to 0.62 of its standard deviation was 4.02e-7 off)
+@pytest.mark.parametrize("M,K,N", [(126, 2048, 512), (3, 4100, 70), (1, 16384, 40), (70, 3001, 33),
+                                   (1, 70000, 33), (250, 2080, 500)])
+@pytest.mark.parametrize("act", [0, 2])
+def test_sgemm_long_k_on_a_short_grid(M, K, N, act):
+    """Error against fp64 as small as the parts of K keep it: 2.4e-7 measured at most (7.3e-7 with
+    16384 in one workgroup's eight parts)."""
+    r = SplitMix64(M + K + N)
+    x, w, b = r.normal((M, K)), r.normal((N, K)), r.normal((N,))
+    out = empty((M, N), np.float32)
+    say("sgemm long k", M, K, N, act)
+    gemm.LaunchSgemm(up(x), up(w), up(b), out, M, K, N, act)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T + b
+    assert _rel(down(out, (M, N)), np.maximum(ref, 0) if act == 2 else ref) <= 4e-7
+
+
+def test_sgemm_long_k_under_capture():
+    """Captured on a stream without a workspace block: the unsplit form, since nothing can be
+    allocated there.  With one: the eager result's bits on every replay."""
+    hip = C.CDLL("libamdhip64.so")
+
+    def ok(rc):
+        assert rc == 0, rc
+
+    M, K, N = 40, 4096, 96
+    r = SplitMix64(4)
+    x, w = r.normal((M, K)), r.normal((N, K))
+    dx, dw, out = up(x), up(w), empty((M, N), np.float32)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+
+    def replays(stream):
+        graph, run = C.c_void_p(), C.c_void_p()
+        h = C.c_void_p(stream.handle)
+        ok(hip.hipStreamBeginCapture(h, 0))
+        gemm.LaunchSgemm(dx, dw, None, out, M, K, N, 0, stream)
+        ok(hip.hipStreamEndCapture(h, C.byref(graph)))
+        ok(hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+        got = []
+        for _ in range(3):
+            out.upload(np.full((M, N), np.nan, np.float32))
+            synchronize()
+            ok(hip.hipGraphLaunch(run, h))
+            got.append(down(out, (M, N)))
+        ok(hip.hipGraphExecDestroy(run))
+        ok(hip.hipGraphDestroy(graph))
+        return got
+
+    say("sgemm long k captured")
+    stream = Stream()
+    for got in replays(stream):
+        assert _rel(got, ref) <= 6e-7  # 3.5e-7 measured unsplit
+    gemm.LaunchSgemm(dx, dw, None, out, M, K, N, 0, stream)
+    eager = down(out, (M, N))
+    for got in replays(stream):
+        np.testing.assert_array_equal(got, eager)
 
 
 def test_sgemm_split_special_values():
