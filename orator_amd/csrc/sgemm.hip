@@ -625,56 +625,78 @@ int launch_sized(const SgemmArgs& a, hipStream_t s) {
   return launch_tile<32, 32, 2, VEC, GLU>(a, s);
 }
 
-// out[i] = act(sum_z part[z][i] + bias), z ascending, or the residual update.
+// out_b[i] = act(sum_z part[z][b][i] + bias), z ascending, or the residual update.
 __global__ __launch_bounds__(256) void sgemm_reduce_kernel(SgemmArgs a, const float* part,
                                                            int splits) {
-  const long MN = static_cast<long>(a.M) * a.N;
+  const long MN = static_cast<long>(a.M) * a.N, all = MN * a.batch;
   const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= MN) return;
+  if (i >= all) return;
   float v = part[i];
-  for (int z = 1; z < splits; ++z) v += part[z * MN + i];
+  for (int z = 1; z < splits; ++z) v += part[z * all + i];
   v = apply_act(v + (a.bias ? a.bias[i % a.N] : 0.0f), a.act);
-  a.out[i] = a.residual ? fmaf(a.res_scale, v, a.out[i]) : v;
+  float* out = a.out + (a.batch > 1 ? i / MN * a.s_out + i % MN : i);
+  *out = a.residual ? fmaf(a.res_scale, v, *out) : v;
 }
 
-// Long K on a short grid: parts of K, 1024 each at least, on workgroups of their own, as many as
-// the CUs take in one round, and a second launch that adds them (us, whole and split: 126 x 2048
-// -> 512 12.0 and 10.1, 1 x 4096 -> 1024 19.0 and 10.7, 64 x 16384 -> 64 65.7 and 13.4; one row and
-// two columns at K = 2^24 63 ms and 0.32).
-int run_split(const SgemmArgs& a, int splits, float* part, hipStream_t s) {
-  const int n_sl = a.K / kSK + (a.K % kSK != 0);
+// Through partial products in memory, for one of two reasons.  Long K on a short grid: parts of K,
+// 1024 each at least, on workgroups of their own, as many as the CUs take in one round, and a
+// second launch that adds them (us, whole and split: 126 x 2048 -> 512 12.0 and 10.1, 1 x 4096 ->
+// 1024 19.0 and 10.7, 64 x 16384 -> 64 65.7 and 13.4; one row and two columns at K = 2^24 63 ms and
+// 0.32).  And outputs that lie over an operand, which other workgroups may still be reading.
+int run_parts(const SgemmArgs& a, int splits, float* part, hipStream_t s) {
   SgemmArgs p = a;
-  p.slices = (n_sl + splits - 1) / splits;
-  splits = (n_sl + p.slices - 1) / p.slices;
-  const long MN = static_cast<long>(a.M) * a.N;
+  if (splits > 1) {
+    const int n_sl = a.K / kSK + (a.K % kSK != 0);
+    p.slices = (n_sl + splits - 1) / splits;
+    splits = (n_sl + p.slices - 1) / p.slices;
+    p.batch = splits;
+  }
+  const long MN = static_cast<long>(a.M) * a.N, all = MN * a.batch;
   p.out = part;
-  p.batch = splits;
   p.s_out = MN;
   p.bias = nullptr;
   p.act = p.residual = 0;
   const bool far = a.K >= 1 << 24;
-  const int rc = a.vec ? (far ? launch_tile<32, 32, 8, true, false, true>(p, s)
-                              : launch_tile<32, 32, 8, true, false>(p, s))
-                       : (far ? launch_tile<32, 32, 8, false, false, true>(p, s)
-                              : launch_tile<32, 32, 8, false, false>(p, s));
+  int rc;
+  if (splits == 1)
+    rc = a.vec ? launch_sized<true, false>(p, s) : launch_sized<false, false>(p, s);
+  else if (a.vec)
+    rc = far ? launch_tile<32, 32, 8, true, false, true>(p, s)
+             : launch_tile<32, 32, 8, true, false>(p, s);
+  else
+    rc = far ? launch_tile<32, 32, 8, false, false, true>(p, s)
+             : launch_tile<32, 32, 8, false, false>(p, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(sgemm_reduce_kernel, dim3(static_cast<unsigned>((MN + 255) / 256)), dim3(256),
-                     0, s, a, part, splits);
+  hipLaunchKernelGGL(sgemm_reduce_kernel, dim3(static_cast<unsigned>((all + 255) / 256)),
+                     dim3(256), 0, s, a, part, splits);
   return check_launch("sgemm_reduce_kernel");
 }
+
+// Whether [p, p + n) and [q, q + m) floats share memory.
+bool overlap(const float* p, long n, const float* q, long m) { return p < q + m && q < p + n; }
 
 int run_sgemm(SgemmArgs a, int batch, bool glu, hipStream_t s) {
   a.batch = batch;
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const long tiles = static_cast<long>((a.M + 31) / 32) * ((a.N + 31) / 32);
-  const long splits = std::min<long>(cus / tiles, a.K / 1024);
-  float* part = nullptr;  // without room for it, as in a capture before the first call: not split
-  if (splits > 1 && batch == 1 && !glu && !a.h16) {
-    const size_t bytes = splits * sizeof(float) * a.M * a.N;
-    if (workspace_at_hand(s, bytes, kWsGemm))
+  long splits = std::min<long>(cus / tiles, a.K / 1024);
+  if (splits < 1 || batch > 1) splits = 1;
+  // operands and outputs of the plain product (of all its batch entries)
+  const bool plain = !glu && !a.group && !a.h16;
+  auto span = [&](long stride, long rows, long cols) { return (batch - 1) * stride + rows * cols; };
+  const long out_n = span(a.s_out, a.M, a.N);
+  const bool over = plain && (overlap(a.out, out_n, a.in, span(a.s_in, a.M, a.K)) ||
+                              overlap(a.out, out_n, a.W, span(a.s_w, a.N, a.K)));
+  float* part = nullptr;
+  if (plain && (splits > 1 || over)) {
+    const size_t bytes = splits * batch * sizeof(float) * a.M * a.N;
+    // without room, as in a capture before the first call, a split product stays whole
+    if (over || workspace_at_hand(s, bytes, kWsGemm)) {
       part = static_cast<float*>(workspace(s, bytes, kWsGemm));
+      if (!part && over) return ORATOR_ERR_HIP;
+    }
   }
-  const int rc = part ? run_split(a, static_cast<int>(splits), part, s)
+  const int rc = part ? run_parts(a, static_cast<int>(splits), part, s)
                  : glu ? launch_sized<true, true>(a, s)
                  : a.vec ? launch_sized<true, false>(a, s) : launch_sized<false, false>(a, s);
   if (rc || !a.ln_g) return rc;

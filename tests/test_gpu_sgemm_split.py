@@ -115,6 +115,23 @@ def test_sgemm_long_k_under_capture():
         np.testing.assert_array_equal(got, eager)
 
 
+@pytest.mark.parametrize("M,K,batch", [(126, 512, 1), (1000, 512, 1), (700, 70, 1), (40, 2048, 1),
+                                       (60, 512, 3)])
+def test_sgemm_output_over_its_operand(M, K, batch):
+    """Output over the input, and over the weight (N = K, M = N): as with an output of its own."""
+    r = SplitMix64(M + K)
+    x, w = r.normal((batch, M, K)), r.normal((batch, K, K))
+    say("sgemm in place", M, K, batch)
+    for over in ("in", "weight"):
+        m = M if over == "in" else K
+        xs = x if over == "in" else r.normal((batch, K, K))
+        dx, dw, want = up(xs), up(w), empty((batch, m, K), np.float32)
+        gemm.LaunchSgemmBatched(dx, dw, want, m, K, K, 2, batch, m * K, K * K, m * K)
+        out = dx if over == "in" else dw
+        gemm.LaunchSgemmBatched(dx, dw, out, m, K, K, 2, batch, m * K, K * K, m * K)
+        np.testing.assert_array_equal(down(out, (batch, m, K)), down(want, (batch, m, K)))
+
+
 def test_sgemm_split_special_values():
     """Rows with an infinity, a NaN, the largest finite value (which rounds past bf16's range), an
     overflowing sum, and operands so small that their bf16 terms are subnormal, beside ordinary
