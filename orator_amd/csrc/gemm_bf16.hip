@@ -8,7 +8,7 @@
 // without any transpose.
 //
 // This register-staged kernel serves what gemm_dma.hip's does not take: K not a multiple of 64, N not
-// of 4, unaligned operands, sizes past 32-bit offsets.
+// of 4, unaligned operands, sizes past 32-bit offsets, outputs over an operand.
 //
 // Workgroup = BM x BN output tile, 4 waves (one per SIMD) in a WGM x WGN grid, each wave
 // (BM/WGM) x (BN/WGN) = FM x FN blocks of 32 x 32 accumulators, two workgroups per CU (73.7 KB
@@ -383,7 +383,8 @@ int launch_tile(const uint16_t* in, const uint16_t* W, const float* bias, float*
 int launch_gemm_bf16_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out, float* tmp,
                             int M, int K, int I, hipStream_t s) {
   if (M <= 0 || K <= 0 || I <= 0) return ORATOR_OK;
-  const bool dma = I % 4 == 0 && gemm_dma_takes(in, W, out, M, K, 2 * I);
+  const size_t out_bytes = 2 * static_cast<size_t>(M) * I;
+  const bool dma = I % 4 == 0 && gemm_dma_takes(in, W, out, out_bytes, M, K, 2 * I);
   if (dma && !gemm_dma_splits(M, K, 2 * I)) return launch_gemm_dma_swiglu(in, W, out, M, K, I, s);
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const long tiles = static_cast<long>((M + 127) / 128) * ((I + 63) / 64);
@@ -409,7 +410,7 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic) {
   if (M <= 0 || K <= 0 || N <= 0) return ORATOR_OK;
-  if (!generic && gemm_dma_takes(in, W, out, M, K, N))
+  if (!generic && gemm_dma_takes(in, W, out, 4 * static_cast<size_t>(M) * N, M, K, N))
     return launch_gemm_dma(in, W, bias, out, M, K, N, act, accumulate, s);
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   auto tiles = [&](int bm, int bn) {

@@ -393,10 +393,17 @@ bool fits32(int M, int K, int N) {
 
 }  // namespace
 
-bool gemm_dma_takes(const void* in, const void* W, const void* out, int M, int K, int N) {
-  const uintptr_t al = reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W) |
-                       reinterpret_cast<uintptr_t>(out);
-  return K % 64 == 0 && N % 4 == 0 && (al & 15u) == 0 && fits32(M, K, N);
+// An output over an operand stays with the register-staged kernel, whose short grids write it from
+// a second launch; here workgroups may still be reading what others write.
+bool gemm_dma_takes(const void* in, const void* W, const void* out, size_t out_bytes, int M, int K,
+                    int N) {
+  const uintptr_t i = reinterpret_cast<uintptr_t>(in), w = reinterpret_cast<uintptr_t>(W),
+                  o = reinterpret_cast<uintptr_t>(out);
+  auto apart = [&](uintptr_t p, long rows) {
+    return p + 2 * rows * K <= o || o + out_bytes <= p;
+  };
+  return K % 64 == 0 && N % 4 == 0 && ((i | w | o) & 15u) == 0 && fits32(M, K, N) && apart(i, M) &&
+         apart(w, N);
 }
 
 int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, float* out, int M,
@@ -414,8 +421,9 @@ bool gemm_dma_takes_f32(const float* in, const void* W, const float* out, int M,
   const uintptr_t ib = reinterpret_cast<uintptr_t>(in), ob = reinterpret_cast<uintptr_t>(out);
   const bool apart = ib + 4 * static_cast<uintptr_t>(M) * K <= ob ||
                      ob + 4 * static_cast<uintptr_t>(M) * N <= ib;
-  return M > 1 && M <= 128 && apart && gemm_dma_takes(in, W, out, M, K, N) && fits32(M, 2 * K, N) &&
-         pick_shape(M, K, N).tile == Tile::k64x64;
+  const size_t out_bytes = 4 * static_cast<size_t>(M) * N;
+  return M > 1 && M <= 128 && apart && gemm_dma_takes(in, W, out, out_bytes, M, K, N) &&
+         fits32(M, 2 * K, N) && pick_shape(M, K, N).tile == Tile::k64x64;
 }
 
 int launch_gemm_dma_f32(const float* in, const uint16_t* W, const float* bias, float* out, int M,

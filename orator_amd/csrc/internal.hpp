@@ -187,8 +187,10 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic = false);
 // The same on tiles loaded straight into LDS (gemm_dma.hip), for the operands gemm_dma_takes: K a
-// multiple of 64, N of 4, 16-byte aligned pointers, 32-bit sizes.  SwiGLU: N = 2I, I a multiple of 4.
-bool gemm_dma_takes(const void* in, const void* W, const void* out, int M, int K, int N);
+// multiple of 64, N of 4, 16-byte aligned pointers, 32-bit sizes, the output apart from the
+// operands.  SwiGLU: N = 2I, I a multiple of 4.
+bool gemm_dma_takes(const void* in, const void* W, const void* out, size_t out_bytes, int M, int K,
+                    int N);
 int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, float* out, int M,
                     int K, int N, int act, bool accumulate, hipStream_t s);
 // The same from fp32 activations, rounded to bf16 inside the kernel; `out` apart from `in`.

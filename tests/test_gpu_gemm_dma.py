@@ -86,3 +86,27 @@ def test_linear_in_place():
     say("linear in place")
     asr_gemm.Linear(buf, up(orc.to_bf16(w)), None, buf, M, K, K, 0)
     np.testing.assert_array_equal(down(buf, (M, K)), x @ w.T)
+
+
+@pytest.mark.parametrize("M,K", [(2, 64), (70, 256), (200, 2048)])
+def test_swiglu_output_over_the_input(M, K):
+    """LinearPreSwiGLU in place (I = K, a grid of fewer tiles than CUs): as with an output apart."""
+    r = np.random.default_rng(M + K)
+    x = orc.to_bf16(r.standard_normal((M, K)).astype(np.float32))
+    w = up(orc.to_bf16((r.standard_normal((2 * K, K)) * K ** -0.5).astype(np.float32)))
+    want, buf = empty((M, K), np.uint16), up(x)
+    say("gemm dma swiglu in place", M, K)
+    asr_gemm.LinearPreSwiGLU(buf, w, want, M, K, K)
+    asr_gemm.LinearPreSwiGLU(buf, w, buf, M, K, K)
+    np.testing.assert_array_equal(down(buf, (M, K), np.uint16), down(want, (M, K), np.uint16))
+
+
+def test_linear_pre_output_over_the_input():
+    """fp32 outputs over the bf16 input (N = K / 2) on a grid whose K is split."""
+    r = np.random.default_rng(11)
+    M, K = 503, 2048
+    x, w = _ints(r, (M, K), 4), _ints(r, (K // 2, K), 4)
+    buf = up(orc.to_bf16(x))
+    say("gemm dma linear pre in place")
+    asr_gemm.LinearPre(buf, up(orc.to_bf16(w)), None, buf, M, K, K // 2, 0)
+    np.testing.assert_array_equal(down(buf, (M, K // 2)), x @ w.T)
