@@ -8,7 +8,8 @@
 // without any transpose.
 //
 // This register-staged kernel serves what gemm_dma.hip's does not take: K not a multiple of 64, N not
-// of 4, unaligned operands, sizes past 32-bit offsets, outputs over an operand.
+// of 4, unaligned operands, sizes past 32-bit offsets, outputs over an operand, and short K
+// with many fp32 outputs.
 //
 // Workgroup = BM x BN output tile, 4 waves (one per SIMD) in a WGM x WGN grid, each wave
 // (BM/WGM) x (BN/WGN) = FM x FN blocks of 32 x 32 accumulators, two workgroups per CU (73.7 KB
@@ -410,7 +411,8 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic) {
   if (M <= 0 || K <= 0 || N <= 0) return ORATOR_OK;
-  if (!generic && gemm_dma_takes(in, W, out, 4 * static_cast<size_t>(M) * N, M, K, N))
+  if (!generic && !gemm_dma_store_bound(M, K, N) &&
+      gemm_dma_takes(in, W, out, 4 * static_cast<size_t>(M) * N, M, K, N))
     return launch_gemm_dma(in, W, bias, out, M, K, N, act, accumulate, s);
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   auto tiles = [&](int bm, int bn) {

@@ -432,6 +432,17 @@ int launch_gemm_dma_f32(const float* in, const uint16_t* W, const float* bias, f
       GemmDmaArgs{in, W, bias, out, nullptr, M, K, N, act, 0, K}, pick_shape(M, K, N).splits, s);
 }
 
+// Short K and many outputs on the larger tiles, whose waves have nothing to do while the tile's stores
+// drain, 32 bytes of 32 rows at a time: the register-staged kernel's are faster as long as rows are
+// whole 128-byte lines, and its sums are in the same order (us, this kernel and that one: 2048 x 64 ->
+// 2048 8.0 and 6.7, 8192 x 128 -> 4096 37.3 and 29.6, 2048 x 192 -> 4096 13.6 and 12.1, 8192 x 256 ->
+// 2048 26.6 and 22.2; 717 x 256 -> 4096 8.1 and 8.0, 8192 x 256 -> 1000 12.7 and 14.0; at K = 512
+// 15 % either way from card to card).
+bool gemm_dma_store_bound(int M, int K, int N) {
+  return K <= 256 && N % 32 == 0 && static_cast<long>(M) * N >= 8192L * K &&
+         pick_shape(M, K, N).tile != Tile::k64x64;
+}
+
 bool gemm_dma_splits(int M, int K, int N) { return pick_shape(M, K, N).splits > 1; }
 
 int launch_gemm_dma_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out, int M, int K,

@@ -197,6 +197,8 @@ int launch_gemm_dma(const uint16_t* in, const uint16_t* W, const float* bias, fl
 bool gemm_dma_takes_f32(const float* in, const void* W, const float* out, int M, int K, int N);
 int launch_gemm_dma_f32(const float* in, const uint16_t* W, const float* bias, float* out, int M,
                         int K, int N, int act, hipStream_t s);
+// Whether launch_gemm_dma takes this shape's products with fp32 outputs more slowly.
+bool gemm_dma_store_bound(int M, int K, int N);
 // Whether launch_gemm_dma splits K for this shape: its sums are then in another order than the
 // unsplit SwiGLU form's.
 bool gemm_dma_splits(int M, int K, int N);
