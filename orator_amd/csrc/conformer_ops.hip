@@ -1,7 +1,7 @@
 // The Conformer layer's non-attention passes (src/model/conformer_layer.cu:28-76,207-246):
 // LayerNorm, GLU (fused with the padding-row mask that follows it), the depthwise time
 // convolution fused with the BatchNorm (eval) + SiLU after it.  (The scaled residual add is the
-// epilogue of the projection before it: launch_sgemm_residual.)
+// epilogue of the projection before it: launch_sgemm_residual_ln.)
 // Each keeps the reference's per-element arithmetic; the fusions only drop the HBM round trips
 // between passes.  All tensors are [T, C] fp32, C the channel count (d_model).
 #include "common.hpp"

@@ -390,7 +390,8 @@ int launch_gemm_bf16_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out
   const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const long tiles = static_cast<long>((M + 127) / 128) * ((I + 63) / 64);
   if (dma || tiles < cus) {
-    if (!tmp) tmp = static_cast<float*>(workspace(s, static_cast<size_t>(M) * 2 * I * sizeof(float)));
+    if (!tmp)
+      tmp = static_cast<float*>(workspace(s, static_cast<size_t>(M) * 2 * I * sizeof(float)));
     if (!tmp) return ORATOR_ERR_HIP;
     if (int rc = launch_gemm_bf16_nt(in, W, nullptr, tmp, M, K, 2 * I, 0, false, s)) return rc;
     return launch_swiglu_bf16(tmp, out, M, I, s);
@@ -403,10 +404,11 @@ int launch_gemm_bf16_swiglu(const uint16_t* in, const uint16_t* W, uint16_t* out
 
 // Tile shape by grid size: 128 x 128 when that grid gives every CU two workgroups, else
 // 128 x 64 (always for `generic`: K not a multiple of 8 or rows not 16-byte aligned, loaded
-// element by element); when even that leaves CUs idle and K is long, K is split over workgroups (partials
-// reduced in a fixed order: deterministic).  Measured at the 503-row prompt shapes: 128 x 64 unsplit
-// beats a K split whenever its grid covers the CUs (qkv, 21.7 vs 23.7 us); below that, splits
-// to two workgroups per CU beat one (down projection, 28.4 vs 36.8 us).
+// element by element); when even that leaves CUs idle and K is long, K is split over workgroups
+// (partials reduced in a fixed order: deterministic).  Measured on this kernel at shapes that
+// gemm_dma.hip takes by now: 128 x 64 unsplit beats a K split whenever its grid covers the CUs (503 x
+// 2048 -> 4096, 21.7 vs 23.7 us); below that, splits to two workgroups per CU beat one (503 x 6144 ->
+// 2048, 28.4 vs 36.8 us).
 int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias, float* out,
                         int M, int K, int N, int act, bool accumulate, hipStream_t s,
                         bool generic) {
@@ -419,7 +421,7 @@ int launch_gemm_bf16_nt(const uint16_t* in, const uint16_t* W, const float* bias
     return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   };
   // 128 x 128 only when every CU gets two of them (one workgroup per CU leaves its epilogue
-  // exposed: the decoder's 2048 x 2048 -> 2048 projections ran 2 % faster on 128 x 64)
+  // exposed: 2048 x 2048 -> 2048 ran 2 % faster on 128 x 64)
   if (!generic && tiles(128, 128) >= 2 * cus)
     return launch_tile<128, 128, 2, 2, 2, false>(in, W, bias, out, M, K, N, act, accumulate, 1, s);
   // when even 128 x 64 tiles leave CUs idle, split K until the grid gives every CU two

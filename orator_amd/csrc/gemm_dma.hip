@@ -1,8 +1,8 @@
 // bf16 GEMM with fp32 accumulation whose tiles go from memory straight into LDS, gfx950:
 // out[M][N] (=|+=) act(in[M][K] W[N][K]^T + bias), and the gate|up form with SwiGLU.
 //
-// Serves every M > 1 product of gemm_bf16.hip's entry points whose K is a multiple of 64 (all of
-// the decoder's and the audio tower's).
+// Serves the M > 1 products of gemm_bf16.hip's entry points whose K is a multiple of 64 (all of the
+// decoder's and the audio tower's), but for short K with many outputs (gemm_dma_store_bound).
 //
 // What bounds it: the matrix cores and LDS bandwidth at once.  A 64 x 64 wave tile reads LDS as
 // long as its MFMAs run (4 KB and 4 MFMAs of 32 cycles per 16 of K, 128 bytes a cycle for 4 waves),
@@ -69,7 +69,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   constexpr int RPA = 64 / CHA, RPW = 64 / CH;  // tile rows per load instruction of a wave
   constexpr int LA = BM / RPA;                 // load instructions of the A tile
   constexpr int L = (LA + BN / RPW) / NW;      // load instructions per wave and stage
-  static_assert(LA % NW == 0 && BN / RPW % NW == 0 && BM % RPA == 0 && BN % RPW == 0 && TM % 32 == 0 && TN % 32 == 0 && NS >= 2 && NS <= 4);
+  static_assert(LA % NW == 0 && BN / RPW % NW == 0 && BM % RPA == 0 && BN % RPW == 0);
+  static_assert(TM % 32 == 0 && TN % 32 == 0 && NS >= 2 && NS <= 4);
   constexpr int kA = BM * CHA * 8;             // the A tile's part of a stage, in 2-byte units
   constexpr int kStage = kA + BN * BK;
   // One array per stage: the compiler's own waits before an LDS read then count the loads into
@@ -94,10 +95,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
   const int M = a.M, N = a.N, K = a.K;
   const int kb = blockIdx.z * a.k_split;
   const int n_k = min(K - kb, a.k_split) / BK;
-  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.A), 0,
-                                                      static_cast<uint32_t>(M) * K * (F32 ? 4 : 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.W), 0,
-                                                      static_cast<uint32_t>(N) * K * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(a.A), 0, static_cast<uint32_t>(M) * K * (F32 ? 4 : 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(a.W), 0, static_cast<uint32_t>(N) * K * 2, 0x00020000);
   // W row of tile row j
   auto w_row = [&](int j) {
     if constexpr (EPI == kDmaSwiglu) {
@@ -186,7 +187,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_bf16_dma_kernel(Gem
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) part_acc[ks % NA][i][j] = mfma32(fb[s][j], fa[s][i], part_acc[ks % NA][i][j]);
+        for (int j = 0; j < FN; ++j)
+          part_acc[ks % NA][i][j] = mfma32(fb[s][j], fa[s][i], part_acc[ks % NA][i][j]);
     }
   };
   auto ready = [&] {  // stage t has arrived for every wave, stage t - 1 is read out
@@ -333,14 +335,20 @@ int launch_tile(GemmDmaArgs a, int splits, hipStream_t s) {
 }
 
 // Tile by the time its rounds over the chip take, in us per 2048 of K (every candidate scales with
-// K alike), measured on 256 CUs:
+// K alike), constants fitted on 256 CUs:
 //   256 x 192, 8 waves, 1 workgroup per CU:             46 a round
 //   128 x 128, 4 waves, 2 stages, 2 workgroups per CU:  36.6 a round, 22 with one per CU
 //   128 x 128, 8 waves, 4 stages, 1 workgroup per CU:   20.1 (the same tile when one per CU is all)
 //   64 x 64, 4 waves, 4 stages, 2 workgroups per CU:    14.4 a round, 11.3 with one per CU
-// so 2048 x 2048 -> 12288 takes the first (92 us; 106 on 128 x 128), 2048 x 2048 -> 4096 the second
-// (36.6; 57 on 64 x 64), 2048 x 6144 -> 2048 the third (59; 65 on the second), 503 x 2048 -> 4096 the
-// last (16.8; 22 on 128 x 128).
+// Every tile at each shape, us of replayed launches on one card, in that order, the rule's last:
+//   2048 x 2048 -> 12288   98.9  103.4  117.6  177.7    99.5
+//   2048 x 2048 -> 4096    44.2   37.2   42.2   57.7    37.1
+//   2048 x 6144 -> 2048    97.8   65.1   52.3   76.5    52.5
+//   1500 x 6144 -> 2048    98.1   62.7   44.4   60.6    44.8
+//   503 x 2048 -> 12288    40.4   31.9   36.7   41.5    32.0
+//   200 x 2048 -> 12288    36.5   24.2   19.2   23.3    18.9
+//   503 x 2048 -> 4096     37.6   21.0   17.5   16.4    16.3
+//   390 x 1024 -> 4096     22.5   12.8   11.4    9.4     9.4
 enum class Tile { k256x192, k128x128, k128x128Deep, k64x64 };
 struct Shape {
   Tile tile;

@@ -215,12 +215,8 @@ int launch_sgemm(const float* in, const float* W, const float* bias, float* out,
                  hipStream_t stream);
 
 // out[M][N] += res_scale * (in W^T + bias): a linear followed by the reference's AddScaledKernel
-// (src/model/conformer_layer.cu:70-76, used at :385, :448, :467, :475), folded into one launch.
-int launch_sgemm_residual(const float* in, const float* W, const float* bias, float* out, int M,
-                          int K, int N, float res_scale, hipStream_t stream);
-
-// launch_sgemm_residual, then ln_out = LayerNorm(out rows; ln_g, ln_b, eps) (conformer_layer.cu:
-// 28-66, the next block's norm); ln_out may be out.
+// (src/model/conformer_layer.cu:70-76, used at :385, :448, :467, :475); then ln_out =
+// LayerNorm(out rows; ln_g, ln_b, eps) (:28-66, the next block's norm); ln_out may be out.
 int launch_sgemm_residual_ln(const float* in, const float* W, const float* bias, float* out,
                              int M, int K, int N, float res_scale, const float* ln_g,
                              const float* ln_b, float* ln_out, float eps, hipStream_t stream);
@@ -242,7 +238,8 @@ int launch_sgemm_group3(const float* in, const float* const W[3], const float* c
                         void* const out[3], int M, int K, int N, int h16_mask,
                         hipStream_t stream);
 
-// out[M][N] = fp16(in W^T), the fp32 product rounded to nearest even once per element: the values an fp16 consumer would round from launch_sgemm's fp32 output.
+// out[M][N] = fp16(in W^T), the fp32 product rounded to nearest even once per element: the values
+// an fp16 consumer would round from launch_sgemm's fp32 output.
 int launch_sgemm_f16_out(const float* in, const float* W, void* out, int M, int K, int N,
                          hipStream_t stream);
 

@@ -729,25 +729,6 @@ int launch_sgemm(const float* in, const float* W, const float* bias, float* out,
   return run_sgemm(a, batch, false, stream);
 }
 
-int launch_sgemm_residual(const float* in, const float* W, const float* bias, float* out, int M,
-                          int K, int N, float res_scale, hipStream_t stream) {
-  if (M <= 0 || N <= 0 || K <= 0) return ORATOR_OK;
-  if (!in || !W || !out) return fail(ORATOR_ERR_INVALID, "sgemm: null pointer");
-  SgemmArgs a{};
-  a.in = in;
-  a.W = W;
-  a.bias = bias;
-  a.out = out;
-  a.M = M;
-  a.K = K;
-  a.N = N;
-  a.residual = 1;
-  a.res_scale = res_scale;
-  a.vec = (K % kSK) == 0 &&
-          ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  return run_sgemm(a, 1, false, stream);
-}
-
 int launch_sgemm_residual_ln(const float* in, const float* W, const float* bias, float* out,
                              int M, int K, int N, float res_scale, const float* ln_g,
                              const float* ln_b, float* ln_out, float eps, hipStream_t stream) {
