@@ -61,8 +61,9 @@ def test_linear_pre_vs_oracle(M, K, N, act, with_bias):
 @pytest.mark.parametrize("M,K,N", [(2048, 2048, 4096), (2048, 2048, 12288), (2048, 6144, 2048)])
 def test_linear_pre_prompt_tiles(M, K, N):
     """The decoder's 2048-token prompt projections (q|k|v 4096, gate|up 12288, down 2048 rows of
-    2048 / 6144): the GEMM's full-grid 128 x 128 path, epilogue without bias (the shapes above
-    take the 128 x 64, split-K and bias / activation paths), same bound."""
+    2048 / 6144): the GEMM's larger tiles (128 x 128 with 4 waves, 256 x 192, 128 x 128 with 8),
+    epilogue without bias (the shapes above take the 64 x 64, split-K and bias / activation
+    paths), same bound."""
     r = SplitMix64(M + K + N)
     x = orc.to_bf16(r.normal((M, K)))
     W = orc.to_bf16(r.normal((N, K), 0.05))
@@ -150,12 +151,14 @@ def test_linear_pre_swiglu_any_k(M, K, I, off):
 
 
 @pytest.mark.parametrize("M,K,I", [(2048, 2048, 6144), (503, 2048, 6144), (300, 1024, 6000),
-                                   (5, 512, 1000), (1, 512, 300)])
+                                   (5, 512, 1000), (1, 512, 300), (2048, 72, 4096),
+                                   (1000, 200, 3000), (90, 200, 1000)])
 def test_linear_pre_swiglu_equals_three_calls(M, K, I):
     """The gate|up GEMM with SwiGLU + bf16 cast in its epilogue is bit-identical to LinearPre
     on the fused [gate; up] weight, SwiGLU and F32ToBf16 (asr_text_decoder.cu:547-552): the
-    fused tile (2048 / 503 rows), a ragged one (300 rows, I = 6000: 64-column tiles cut at
-    the edge), the short-grid path (5 rows) and the GEMV path (1 row)."""
+    direct-to-LDS kernel's tiles (2048 to 5 rows; I = 6000 and 1000 cut at the edge), the GEMV
+    path (1 row), and for K not a multiple of 64 the register-staged kernel's fused tile (2048
+    rows, 1000 ragged ones) and its short grid (90 rows)."""
     from orator_amd import asr_ops
     r = SplitMix64(M + 3 * K + I)
     x = orc.to_bf16(r.normal((M, K)))

@@ -20,13 +20,13 @@ def _ints(r, shape, lim):
 # 64 x 64 tiles: one row pair, ragged rows and columns, one K step, fewer steps than stages, uneven K
 # splits; 128 x 128 with 4 stages (one tile per CU at most); 128 x 128 with 2; 256 x 192; K not a
 # multiple of 64 and N not of 4 (the register-staged kernel) beside them, and the short K with many
-# outputs that go to it too
+# outputs that go to it too; its 128 x 128 tiles last
 @pytest.mark.parametrize("M,K,N", [(2, 64, 4), (63, 128, 60), (65, 192, 68), (130, 320, 516),
                                    (3, 2048, 2044), (65, 4160, 1000), (503, 4160, 2048),
                                    (2000, 64, 2044), (1921, 320, 2044), (2000, 64, 4092),
                                    (1921, 192, 4036), (2040, 64, 12284), (1793, 192, 12100),
                                    (130, 72, 516), (130, 64, 514), (2040, 64, 2048),
-                                   (1921, 256, 4096)])
+                                   (1921, 256, 4096), (2040, 72, 4100), (1921, 200, 6004)])
 @pytest.mark.parametrize("bias,act", [(False, 0), (True, 2)])
 def test_gemm_dma_exact(M, K, N, bias, act):
     r = np.random.default_rng(M + K + N)
