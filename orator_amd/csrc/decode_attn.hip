@@ -1218,7 +1218,7 @@ constexpr long kFuseMaxWorkgroups = 2048;
 static_assert(kFuseMaxWorkgroups <= kArriveCounters, "a fused launch has B * Hkv <= its splits");
 
 // Split length: 128 keys (one 32-key chunk per wave, 117 VGPRs, 4 waves/SIMD), measured
-// ahead of 256 (2 waves/SIMD) on every configs[2] case: B = 16 at 1K/2K/4K keys by 4-5%, a
+// ahead of 256 (2 waves/SIMD) on every case of the decode sweep: B = 16 at 1K/2K/4K keys by 4-5%, a
 // single stream by 6-23%.  G = 4 keeps 4 heads of state per lane and runs 256-key splits.
 int choose_split(int /*B*/, int /*Hkv*/, int G, int /*capacity*/) {
   if (G == 4) return 256;  // the only G = 4 instantiation (launch_dh_g)

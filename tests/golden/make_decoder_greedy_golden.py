@@ -1,5 +1,5 @@
-"""Writes tests/golden/decoder_greedy_c5.npz: the oracle's greedy decode of BASELINE
-configs[4] (the 28-layer Qwen3-ASR-shaped decoder, random bf16 weights, 2048-row prefill of
+"""Writes tests/golden/decoder_greedy_c5.npz: the oracle's greedy decode of the full
+synthetic decoder (28 layers, Qwen3-ASR-shaped, random bf16 weights, 2048-row prefill of
 N(0, 0.02) embeddings, 256 greedy steps, EOS off), for tests/test_gpu_decoder_c5.py.
 
 Run (CPU, ~10 min on 8 cores):  python tests/golden/make_decoder_greedy_golden.py

@@ -90,9 +90,9 @@ def _to_f16_bits(x):
                                              (1, 1, True), (33, 20, True), (300, 300, False),
                                              (40, 0, True), (70, 0, False), (1500, 1500, True)])
 def test_relpos_fused_vs_oracle(T, valid, in_f16):
-    """Fused fp16-MFMA rel-pos attention (BASELINE configs[3]: fp16 inputs N(0,1)).  fp16
+    """Fused fp16-MFMA rel-pos attention (fp16 inputs N(0,1)).  fp16
     operands with fp32 accumulation: max abs error <= 2e-2 on unit-scale outputs (the
-    north_star's bf16/fp16 bar), judged against the oracle run on the fp16-rounded inputs; and
+    bar of the 16-bit modes), judged against the oracle run on the fp16-rounded inputs; and
     within 2x (+2e-5) of the error the kernel's own fp16 roundings predict (tests/fp16_model.py,
     computed before the device runs: ~6e-4 at T = 717)."""
     H, Dk = 8, 64

@@ -1,4 +1,4 @@
-"""GPU parity of BASELINE configs[4]: greedy token ids of the full synthetic decoder (28
+"""GPU parity of the greedy token ids of the full synthetic decoder (28
 layers, hidden 2048, 16/8 heads, SwiGLU 6144, vocab 151936, tied lm_head, random bf16 weights,
 2048-row prefill of N(0, 0.02) embeddings, 256 greedy steps, EOS off) against the oracle's
 (tests/golden/decoder_greedy_c5.npz, written by tests/golden/make_decoder_greedy_golden.py

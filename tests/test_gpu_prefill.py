@@ -1,7 +1,7 @@
 """GPU parity: MFMA prefill attention against the oracle's GqaCacheAttnKernel restatement.
 
 fp32 mode: max |g - r| / max(|r|, 0.05) <= 1e-4.  bf16 mode: max |g - r| <= 2e-2 on
-unit-scale outputs.  Inputs follow BASELINE configs[1]: N(0,1) q/k/v, QK-RMSNorm (unit
+unit-scale outputs.  Inputs: N(0,1) q/k/v, QK-RMSNorm (unit
 gain, eps 1e-6) and RoPE theta 1e6 at the tokens' absolute positions, K/V rounded to bf16
 by the KV write."""
 from __future__ import annotations
@@ -60,7 +60,7 @@ def _run(q, kc, vc, pos0, cap, mode, Hkv, page=None):
 
 @pytest.mark.parametrize("mode", [da.PREFILL_FP32, da.PREFILL_BF16])
 def test_prefill_config2_shape(mode):
-    """BASELINE configs[1]: T = 503 (128 prompt + 375 audio), pos0 = 0."""
+    """T = 503 (128 prompt + 375 audio), pos0 = 0."""
     T, Hq, Hkv, Dh = 503, 16, 8, 128
     q, kc, vc = _layer_inputs(503, T, 0)
     ref = orc.gqa_prefill(q, kc, vc, 0, 1.0 / math.sqrt(Dh), threads=8)
